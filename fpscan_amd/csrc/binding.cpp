@@ -117,8 +117,10 @@ void* launch_stream(const at::Tensor& like) {
   return stream;
 }
 
-at::Tensor fullscan_forward(const at::Tensor& Ax, const at::Tensor& Bx, const at::Tensor& out,
-                            bool reverse) {
+// The forward or reverse scan; `saved`: the forward of a training step, whose gates and output
+// the backward will read (fpscan_scan_fwd_saved).
+at::Tensor run_forward(const at::Tensor& Ax, const at::Tensor& Bx, const at::Tensor& out,
+                       bool reverse, bool saved) {
   check_input(Ax, "Ax");
   check_input(Bx, "Bx");
   check_like(Ax, Bx, "Ax", "Bx");
@@ -136,11 +138,24 @@ at::Tensor fullscan_forward(const at::Tensor& Ax, const at::Tensor& Bx, const at
   const int dt = dtype_code(Bx.scalar_type());
   const size_t ws_bytes = fpscan_workspace_bytes(Bx.size(0), D, L, dt, FPSCAN_OP_FWD);
   at::Tensor ws = workspace(ws_bytes, Bx);
-  const int status = fpscan_scan_fwd(Ax.data_ptr(), Bx.data_ptr(), out.data_ptr(), Bx.size(0),
-                                     D, L, D * L, L, dt, reverse ? 1 : 0,
-                                     ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, stream);
+  void* w = ws_bytes ? ws.data_ptr() : nullptr;
+  const int status =
+      saved ? fpscan_scan_fwd_saved(Ax.data_ptr(), Bx.data_ptr(), out.data_ptr(), Bx.size(0), D,
+                                    L, D * L, L, dt, w, ws_bytes, stream)
+            : fpscan_scan_fwd(Ax.data_ptr(), Bx.data_ptr(), out.data_ptr(), Bx.size(0), D, L,
+                              D * L, L, dt, reverse ? 1 : 0, w, ws_bytes, stream);
   check_status(status);
   return out;
+}
+
+at::Tensor fullscan_forward(const at::Tensor& Ax, const at::Tensor& Bx, const at::Tensor& out,
+                            bool reverse) {
+  return run_forward(Ax, Bx, out, reverse, false);
+}
+
+at::Tensor fullscan_forward_saved(const at::Tensor& Ax, const at::Tensor& Bx,
+                                  const at::Tensor& out) {
+  return run_forward(Ax, Bx, out, false, true);
 }
 
 std::tuple<at::Tensor, at::Tensor> fullscan_backward(const at::Tensor& gates,
@@ -185,7 +200,7 @@ struct PScanFunction : public torch::autograd::Function<PScanFunction> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& gates,
                             const at::Tensor& tokens) {
     at::Tensor out = at::empty_like(tokens);
-    fullscan_forward(gates, tokens, out, false);
+    run_forward(gates, tokens, out, false, gates.requires_grad() || tokens.requires_grad());
     ctx->save_for_backward({gates, out});
     return out;
   }
@@ -329,9 +344,9 @@ void check_rate(const at::Tensor& rate, const at::Tensor& like, const char* name
               " float32 tensor with one value per dim (", like.size(1), "), got ", rate.sizes());
 }
 
-at::Tensor fullscan_forward_softplus(const at::Tensor& z, const at::Tensor& rate,
-                                     const at::Tensor& tokens, const at::Tensor& out,
-                                     bool reverse) {
+at::Tensor run_forward_softplus(const at::Tensor& z, const at::Tensor& rate,
+                                const at::Tensor& tokens, const at::Tensor& out, bool reverse,
+                                bool saved) {
   check_input(z, "z");
   check_input(tokens, "tokens");
   check_like(z, tokens, "z", "tokens");
@@ -344,11 +359,27 @@ at::Tensor fullscan_forward_softplus(const at::Tensor& z, const at::Tensor& rate
   c10::hip::HIPGuardMasqueradingAsCUDA guard(tokens.device());
   void* stream = launch_stream(tokens);
   const int64_t D = tokens.size(1), L = tokens.size(2);
-  const int status = fpscan_scan_fwd_softplus(
-      z.data_ptr(), rate.data_ptr<float>(), tokens.data_ptr(), out.data_ptr(), tokens.size(0),
-      D, L, D * L, L, dtype_code(tokens.scalar_type()), reverse ? 1 : 0, stream);
+  const int dt = dtype_code(tokens.scalar_type());
+  const int status =
+      saved ? fpscan_scan_fwd_softplus_saved(z.data_ptr(), rate.data_ptr<float>(),
+                                             tokens.data_ptr(), out.data_ptr(), tokens.size(0),
+                                             D, L, D * L, L, dt, stream)
+            : fpscan_scan_fwd_softplus(z.data_ptr(), rate.data_ptr<float>(), tokens.data_ptr(),
+                                       out.data_ptr(), tokens.size(0), D, L, D * L, L, dt,
+                                       reverse ? 1 : 0, stream);
   check_status(status);
   return out;
+}
+
+at::Tensor fullscan_forward_softplus(const at::Tensor& z, const at::Tensor& rate,
+                                     const at::Tensor& tokens, const at::Tensor& out,
+                                     bool reverse) {
+  return run_forward_softplus(z, rate, tokens, out, reverse, false);
+}
+
+at::Tensor fullscan_forward_softplus_saved(const at::Tensor& z, const at::Tensor& rate,
+                                           const at::Tensor& tokens, const at::Tensor& out) {
+  return run_forward_softplus(z, rate, tokens, out, false, true);
 }
 
 void fullscan_backward_softplus(const at::Tensor& z, const at::Tensor& rate,
@@ -407,6 +438,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fullscan_forward", &fullscan_forward,
         "first-order linear-recurrence scan, forward or reverse, written into out (HIP, gfx950)",
         pybind11::arg("Ax"), pybind11::arg("Bx"), pybind11::arg("out"), pybind11::arg("reverse"));
+  m.def("fullscan_forward_saved", &fullscan_forward_saved,
+        "fullscan_forward for a training step: the same results, with the gates and the output "
+        "left in the memory-side cache for the backward", pybind11::arg("Ax"),
+        pybind11::arg("Bx"), pybind11::arg("out"));
   m.def("fullscan_backward", &fullscan_backward,
         "fused backward of the forward scan: (grad_gates, grad_tokens) (HIP, gfx950)",
         pybind11::arg("gates"), pybind11::arg("out"), pybind11::arg("grad_out"),
@@ -425,6 +460,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "scan with gates exp(-softplus(z) * rate[d]) computed on load, written into out",
         pybind11::arg("z"), pybind11::arg("rate"), pybind11::arg("tokens"), pybind11::arg("out"),
         pybind11::arg("reverse"));
+  m.def("fullscan_forward_softplus_saved", &fullscan_forward_softplus_saved,
+        "fullscan_forward_softplus for a training step (see fullscan_forward_saved)",
+        pybind11::arg("z"), pybind11::arg("rate"), pybind11::arg("tokens"), pybind11::arg("out"));
   m.def("fullscan_backward_softplus", &fullscan_backward_softplus,
         "fused backward of the softplus-gate scan: writes grad_z, grad_tokens and one "
         "d loss / d rate partial per row", pybind11::arg("z"), pybind11::arg("rate"),

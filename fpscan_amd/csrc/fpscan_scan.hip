@@ -127,12 +127,12 @@ struct RowRsrc {
 // sub-chunk inside the row, or kNoOffset for a ring slot past the end of the row (the loads
 // are still issued so that the wait counts stay static). Boundary values read outside the
 // row come back as 0 and are replaced by the identity where they are used.
-template <class E, int kMode>
+template <class E, int kMode, int kKeep = kKeepNone>
 __device__ __forceinline__ void load_slot(const RowRsrc<kMode>& rr, Slot<kMode>& s,
                                           uint32_t sub_bytes, uint32_t lane_off) {
   constexpr int kSubBytes = 64 * 16;
   const uint32_t off = sub_bytes + lane_off;
-  s.v[0] = bld16(rr.in0, off);
+  s.v[0] = bld16<gate_policy(kKeep)>(rr.in0, off);
   s.v[1] = bld16(rr.in1, off);
   if constexpr (kMode == kBwd) {
     s.v[2] = bld16(rr.in2, off);
@@ -347,7 +347,8 @@ __device__ __forceinline__ float segment_sum(float v, int sl) {
 // Long rows: W waves per row, U sub-chunks in flight per wave.
 // ---------------------------------------------------------------------------------------
 // R: rows per block when W == 1 (one wave per row), 1 otherwise.
-template <class E, int kMode, int W, int U, class Gp = GatePlain, int R = (W == 1 ? 4 : 1)>
+template <class E, int kMode, int W, int U, class Gp = GatePlain, int R = (W == 1 ? 4 : 1),
+          int kKeep = kKeepNone>
 __global__ void __launch_bounds__(W == 1 ? 64 * R : 64 * W) scan_long_rows(const Args a) {
   constexpr int V = E::V;
   constexpr int kSub = 64 * V;
@@ -392,7 +393,7 @@ __global__ void __launch_bounds__(W == 1 ? 64 * R : 64 * W) scan_long_rows(const
     Slot<kMode> ring[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      load_slot<E, kMode>(rr, ring[u], sub_bytes(u), lane_off);
+      load_slot<E, kMode, kKeep>(rr, ring[u], sub_bytes(u), lane_off);
       __builtin_amdgcn_sched_barrier(0);  // slot u's loads before slot u+1's (wait counts)
     }
 
@@ -453,10 +454,10 @@ __global__ void __launch_bounds__(W == 1 ? 64 * R : 64 * W) scan_long_rows(const
         const float y_enter = dpp<kWaveShr1>(c_in, y_lane_end);
         u32x4 o0, o1;
         finish_lane<E, kMode, Gp>(al, be, ysh, y_enter, o0, o1, &aux, &rate_sum);
-        bst16(rr.out0, sb + lane_off, o0);
+        bst16<out_policy(kKeep)>(rr.out0, sb + lane_off, o0);
         if constexpr (kMode == kBwd) bst16(rr.out1, sb + lane_off, o1);
         const uint32_t next = (r + U < nrounds) ? sub_bytes(r + U) : kNoOffset;
-        load_slot<E, kMode>(rr, ring[u], next, lane_off);
+        load_slot<E, kMode, kKeep>(rr, ring[u], next, lane_off);
         // keep the ring order: without this the scheduler hoists the next slot's arithmetic
         // above this slot's refill, which turns every wait into a wait for all loads
         __builtin_amdgcn_sched_barrier(0);
@@ -991,10 +992,12 @@ int launch(const void* kernel, int64_t groups, int threads, const Args& a, hipSt
   return err == hipSuccess ? FPSCAN_OK : FPSCAN_ERR_LAUNCH;
 }
 
-template <class E, int kMode, int W, class Gp>
+template <class E, int kMode, int W, class Gp, int kKeep>
 const void* long_kernel(int u) {
   if constexpr (W == 1) {
-    if (u >= 4) return reinterpret_cast<const void*>(&scan_long_rows<E, kMode, W, 4, Gp>);
+    if (u >= 4)
+      return reinterpret_cast<const void*>(
+          &scan_long_rows<E, kMode, W, 4, Gp, W == 1 ? 4 : 1, kKeep>);
   }
   // W = 16 keeps three sub-chunks in flight per wave: measured 2-5 % faster than two on
   // rows of 4 or more rounds (bf16 B8 D1024 L65536 forward 552 us against 568, backward 928
@@ -1006,23 +1009,26 @@ const void* long_kernel(int u) {
   // VGPRs in bf16, no spills, the same one workgroup per CU) it measured within 0.5 % of two
   // in bf16 and fp32 at (8, 1024, 65536), (2, 512, 65536) and (4, 256, 32768).
   if constexpr (W == 16 && kMode != kBwd) {
-    if (u >= 4) return reinterpret_cast<const void*>(&scan_long_rows<E, kMode, W, 4, Gp>);
+    if (u >= 4)
+      return reinterpret_cast<const void*>(
+          &scan_long_rows<E, kMode, W, 4, Gp, W == 1 ? 4 : 1, kKeep>);
   }
   if constexpr (W == 16 && (!Gp::kFused || kMode != kBwd)) {
-    if (u >= 3) return reinterpret_cast<const void*>(&scan_long_rows<E, kMode, W, 3, Gp>);
+    if (u >= 3) return reinterpret_cast<const void*>(&scan_long_rows<E, kMode, W, 3, Gp, 1, kKeep>);
   }
-  if (u >= 2) return reinterpret_cast<const void*>(&scan_long_rows<E, kMode, W, 2, Gp>);
-  return reinterpret_cast<const void*>(&scan_long_rows<E, kMode, W, 1, Gp>);
+  constexpr int R = W == 1 ? 4 : 1;
+  if (u >= 2) return reinterpret_cast<const void*>(&scan_long_rows<E, kMode, W, 2, Gp, R, kKeep>);
+  return reinterpret_cast<const void*>(&scan_long_rows<E, kMode, W, 1, Gp, R, kKeep>);
 }
 
-template <class E, int kMode, class Gp>
+template <class E, int kMode, class Gp, int kKeep>
 const void* long_kernel(int w, int u) {
   switch (w) {
-    case 1: return long_kernel<E, kMode, 1, Gp>(u);
-    case 2: return long_kernel<E, kMode, 2, Gp>(u);
-    case 4: return long_kernel<E, kMode, 4, Gp>(u);
-    case 8: return long_kernel<E, kMode, 8, Gp>(u);
-    default: return long_kernel<E, kMode, 16, Gp>(u);
+    case 1: return long_kernel<E, kMode, 1, Gp, kKeep>(u);
+    case 2: return long_kernel<E, kMode, 2, Gp, kKeep>(u);
+    case 4: return long_kernel<E, kMode, 4, Gp, kKeep>(u);
+    case 8: return long_kernel<E, kMode, 8, Gp, kKeep>(u);
+    default: return long_kernel<E, kMode, 16, Gp, kKeep>(u);
   }
 }
 
@@ -1072,7 +1078,7 @@ int run_tiled(const Args& a, const TilePlan& plan, void* workspace, hipStream_t 
 
 // Fused-gate calls (Gp = GateSoftplus) always stream rows: the tiled kernel rebuilds a tile's
 // maps at its deferred finish, which would evaluate the gate transform twice.
-template <class E, int kMode, class Gp = GatePlain>
+template <class E, int kMode, class Gp, int kKeep>
 int run(const Args& a, void* workspace, size_t ws_bytes, hipStream_t stream) {
   constexpr int V = E::V;
   constexpr int kSub = 64 * V;
@@ -1134,21 +1140,48 @@ int run(const Args& a, void* workspace, size_t ws_bytes, hipStream_t stream) {
     // The fused-gate kernels gain as much (fp32 config 5 shape forward 125.6 -> 121.6 us,
     // backward 224.4 -> 208.7; bf16 (64, 4096, 512) 133.3 / 223.9 -> 121.6 / 213.8).
     if (nsub == 1 && ow == 0 && ou == 0 && a.rows >= (kMode == kBwd ? 64 << 10 : 32 << 10))
-      return launch(reinterpret_cast<const void*>(&scan_long_rows<E, kMode, 1, 1, Gp, 1>),
+      return launch(reinterpret_cast<const void*>(&scan_long_rows<E, kMode, 1, 1, Gp, 1, kKeep>),
                     a.rows, 64, a, stream);
-    return launch(long_kernel<E, kMode, Gp>(1, u), (a.rows + 3) / 4, 256, a, stream);
+    return launch(long_kernel<E, kMode, Gp, kKeep>(1, u), (a.rows + 3) / 4, 256, a, stream);
   }
-  return launch(long_kernel<E, kMode, Gp>(w, u), a.rows, 64 * w, a, stream);
+  return launch(long_kernel<E, kMode, Gp, kKeep>(w, u), a.rows, 64 * w, a, stream);
 }
 
-template <int kMode, class Gp = GatePlain>
+template <int kMode, class Gp = GatePlain, int kKeep = kKeepNone>
 int dispatch(int dtype, const Args& a, void* ws, size_t ws_bytes, hipStream_t stream) {
   switch (dtype) {
-    case FPSCAN_DTYPE_F32: return run<F32, kMode, Gp>(a, ws, ws_bytes, stream);
-    case FPSCAN_DTYPE_F16: return run<F16, kMode, Gp>(a, ws, ws_bytes, stream);
-    case FPSCAN_DTYPE_BF16: return run<BF16, kMode, Gp>(a, ws, ws_bytes, stream);
+    case FPSCAN_DTYPE_F32: return run<F32, kMode, Gp, kKeep>(a, ws, ws_bytes, stream);
+    case FPSCAN_DTYPE_F16: return run<F16, kMode, Gp, kKeep>(a, ws, ws_bytes, stream);
+    case FPSCAN_DTYPE_BF16: return run<BF16, kMode, Gp, kKeep>(a, ws, ws_bytes, stream);
     default: return FPSCAN_ERR_DTYPE;
   }
+}
+
+// What the forward of a training step leaves in the 256 MiB memory-side cache for its
+// backward (kKeepBoth / kKeepOut, see scan_common.h), while the gates and the output fit there
+// together (a tensor of at most 128 MiB). Measured on MI355X, a training step over three sets
+// of tensors in turn, streamed -> output kept / both kept (us): bf16 (1, 1024, 65536), 128 MiB,
+// 198.9 -> 182.8 / 170.8; fp32 (2, 256, 65536) 193.3 -> 180.7 / 167.6; bf16 (4, 1024, 8192), 64
+// MiB, 89.5 -> 86.8 / 84.4; bf16 (8, 2048, 2048) 89.3 -> 88.2 / 83.8. Right after the inputs
+// were written, which leaves them in that cache: 203 -> 191.5 / 185.6 at 128 MiB and 91.9 ->
+// 90.6 / 86.9 at 64. With the cache full of other data still to be written back, lines that
+// are kept have to push it out: even at 128 MiB (207 -> 205 / 208), 96 -> 97.5 / 101.4 at 64. Above 128
+// MiB keeping pays only part of the time (256 MiB fp32 (64, 4096, 256): 326 -> 303 with the
+// gates kept, but 337 -> 352 with the cache full; bf16 (2, 1024, 65536) 362 -> 375 with both),
+// so those stream. With the softplus gates only the output is kept (128 MiB 183.3 -> 180.2, 64
+// MiB fp32 93.1 -> 91.7): keeping z as well measured 8 % slower with the cache full. A forward
+// alone gains nothing (138.5 us streamed, 144.5 with both at 256 MiB), so fpscan_scan_fwd
+// streams, and so do rows shorter than a sub-chunk (keeping measured 2 % slower at 128 MiB,
+// bf16 (64, 8192, 128)).
+constexpr int64_t kKeepMaxBytes = 128ll << 20;
+
+template <class Gp>
+int dispatch_saved(int dtype, int size, const Args& a, void* ws, size_t ws_bytes,
+                   hipStream_t stream) {
+  constexpr int kKeep = Gp::kFused ? kKeepOut : kKeepBoth;
+  return a.rows * a.seqlen * size <= kKeepMaxBytes
+             ? dispatch<kFwd, Gp, kKeep>(dtype, a, ws, ws_bytes, stream)
+             : dispatch<kFwd, Gp>(dtype, a, ws, ws_bytes, stream);
 }
 
 int itemsize(int dtype) {
@@ -1266,6 +1299,22 @@ int fpscan_scan_fwd(const void* gates, const void* tokens, void* out, int64_t ba
                  : dispatch<kFwd>(dtype, a, workspace, workspace_bytes, s);
 }
 
+int fpscan_scan_fwd_saved(const void* gates, const void* tokens, void* out, int64_t batch,
+                          int64_t dim, int64_t seqlen, int64_t stride_b, int64_t stride_d,
+                          int dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  Args a{};
+  const int st = validate(batch, dim, seqlen, stride_b, stride_d, dtype, &a);
+  if (st != FPSCAN_OK) return st;
+  if (a.rows == 0) return FPSCAN_OK;
+  if (!gates || !tokens || !out) return FPSCAN_ERR_NULL;
+  if (!aligned16(gates) || !aligned16(tokens) || !aligned16(out)) return FPSCAN_ERR_ALIGN;
+  a.in0 = gates;
+  a.in1 = tokens;
+  a.out0 = out;
+  return dispatch_saved<GatePlain>(dtype, itemsize(dtype), a, workspace, workspace_bytes,
+                                   static_cast<hipStream_t>(stream));
+}
+
 int fpscan_scan_bwd(const void* gates, const void* out, const void* grad_out, void* grad_gates,
                     void* grad_tokens, int64_t batch, int64_t dim, int64_t seqlen,
                     int64_t stride_b, int64_t stride_d, int dtype, void* workspace,
@@ -1309,24 +1358,43 @@ int fpscan_scan_fwd_noalloc(const void* gates, const void* tokens, void* out, in
                  : dispatch<kFwd>(dtype, a, ws, sizeof(scratch), s);
 }
 
-int fpscan_scan_fwd_softplus(const void* z, const float* rate, const void* tokens, void* out,
-                             int64_t batch, int64_t dim, int64_t seqlen, int64_t stride_b,
-                             int64_t stride_d, int dtype, int reverse, void* stream) {
-  Args a{};
-  const int st = validate(batch, dim, seqlen, stride_b, stride_d, dtype, &a);
-  if (st != FPSCAN_OK) return st;
-  if (a.rows == 0) return FPSCAN_OK;
+static int softplus_args(const void* z, const float* rate, const void* tokens, void* out,
+                         int64_t batch, int64_t dim, int64_t seqlen, int64_t stride_b,
+                         int64_t stride_d, int dtype, Args* a) {
+  const int st = validate(batch, dim, seqlen, stride_b, stride_d, dtype, a);
+  if (st != FPSCAN_OK || a->rows == 0) return st;
   if (!z || !rate || !tokens || !out) return FPSCAN_ERR_NULL;
   if (!aligned16(z) || !aligned16(tokens) || !aligned16(out) ||
       (reinterpret_cast<uintptr_t>(rate) & 3u) != 0)
     return FPSCAN_ERR_ALIGN;
-  a.in0 = z;
-  a.in1 = tokens;
-  a.out0 = out;
-  a.rate = rate;
+  a->in0 = z;
+  a->in1 = tokens;
+  a->out0 = out;
+  a->rate = rate;
+  return FPSCAN_OK;
+}
+
+int fpscan_scan_fwd_softplus(const void* z, const float* rate, const void* tokens, void* out,
+                             int64_t batch, int64_t dim, int64_t seqlen, int64_t stride_b,
+                             int64_t stride_d, int dtype, int reverse, void* stream) {
+  Args a{};
+  const int st = softplus_args(z, rate, tokens, out, batch, dim, seqlen, stride_b, stride_d,
+                               dtype, &a);
+  if (st != FPSCAN_OK || a.rows == 0) return st;
   hipStream_t s = static_cast<hipStream_t>(stream);
   return reverse ? dispatch<kRev, GateSoftplus>(dtype, a, nullptr, 0, s)
                  : dispatch<kFwd, GateSoftplus>(dtype, a, nullptr, 0, s);
+}
+
+int fpscan_scan_fwd_softplus_saved(const void* z, const float* rate, const void* tokens,
+                                   void* out, int64_t batch, int64_t dim, int64_t seqlen,
+                                   int64_t stride_b, int64_t stride_d, int dtype, void* stream) {
+  Args a{};
+  const int st = softplus_args(z, rate, tokens, out, batch, dim, seqlen, stride_b, stride_d,
+                               dtype, &a);
+  if (st != FPSCAN_OK || a.rows == 0) return st;
+  return dispatch_saved<GateSoftplus>(dtype, itemsize(dtype), a, nullptr, 0,
+                                      static_cast<hipStream_t>(stream));
 }
 
 int fpscan_scan_bwd_softplus(const void* z, const float* rate, const void* out,

@@ -112,14 +112,28 @@ __device__ __forceinline__ Rsrc row_rsrc(const void* p, int64_t row_base, int si
       const_cast<char*>(static_cast<const char*>(p)) + row_base * size, (short)0, bytes, kRsrcWord3);
 }
 
-// Every element is read once: the 16-byte operand loads are nontemporal, like the stores.
+// Every element is read once: the 16-byte operand loads are nontemporal, like the stores,
+// unless a kernel names another policy (0: the default one, which leaves the lines in the
+// memory-side cache).
+template <int kPolicy = kCacheNT>
 __device__ __forceinline__ u32x4 bld16(Rsrc r, uint32_t off) {
-  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, kCacheNT));
+  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, kPolicy));
 }
 
+template <int kPolicy = kCacheNT>
 __device__ __forceinline__ void bst16(Rsrc r, uint32_t off, u32x4 v) {
-  __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, kCacheNT);
+  __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, kPolicy);
 }
+
+// What a forward leaves in the 256 MiB memory-side cache for the backward that reads its
+// output and its gates again: nothing (both are streamed), the output, or both. Chosen on the
+// host (dispatch_saved).
+constexpr int kKeepNone = 0;
+constexpr int kKeepOut = 1;
+constexpr int kKeepBoth = 2;
+
+constexpr int gate_policy(int keep) { return keep == kKeepBoth ? 0 : kCacheNT; }
+constexpr int out_policy(int keep) { return keep != kKeepNone ? 0 : kCacheNT; }
 
 // Byte offset that no row range contains: loads from it return 0 without touching memory.
 constexpr uint32_t kNoOffset = 0x80000000u;

@@ -94,7 +94,8 @@ class PScan(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, gates: torch.Tensor, tokens: torch.Tensor) -> torch.Tensor:
-        out = scan_forward(gates, tokens)
+        out = torch.empty_like(tokens)
+        _load_extension().fullscan_forward_saved(gates, tokens, out)
         ctx.save_for_backward(gates, out)
         return out
 
@@ -219,7 +220,8 @@ class PScanSoftplus(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, z: torch.Tensor, rate: torch.Tensor, tokens: torch.Tensor) -> torch.Tensor:
-        out = scan_forward_softplus(z, rate, tokens)
+        out = torch.empty_like(tokens)
+        _load_extension().fullscan_forward_softplus_saved(z, rate, tokens, out)
         ctx.save_for_backward(z, rate, out)
         return out
 

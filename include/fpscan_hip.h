@@ -114,6 +114,15 @@ int fpscan_scan_fwd_noalloc(const void* gates, const void* tokens, void* out,
                             int64_t stride_b, int64_t stride_d,
                             int dtype, int reverse, void* stream);
 
+/* The forward of a training step: fpscan_scan_fwd's forward direction, with the same results,
+ * for a caller that will hand `gates` and `out` to fpscan_scan_bwd. Up to 128 MiB per tensor it
+ * reads the gates and writes the output with the cache policy that leaves them in the 256 MiB
+ * memory-side cache instead of streaming them past it. Same workspace as fpscan_scan_fwd. */
+int fpscan_scan_fwd_saved(const void* gates, const void* tokens, void* out,
+                          int64_t batch, int64_t dim, int64_t seqlen,
+                          int64_t stride_b, int64_t stride_d, int dtype,
+                          void* workspace, size_t workspace_bytes, void* stream);
+
 /* Fused backward of the forward scan, given the saved forward output `out`.
  * Replaces the composition in PScan.backward (fpscan/ops.py:69-83): shifted-gate copy,
  * reverse scan (full_scan.cu:198-200), shifted-output copy and the product, in one pass
@@ -184,6 +193,13 @@ int fpscan_scan_fwd_softplus(const void* z, const float* rate, const void* token
                              int64_t batch, int64_t dim, int64_t seqlen,
                              int64_t stride_b, int64_t stride_d,
                              int dtype, int reverse, void* stream);
+
+/* fpscan_scan_fwd_softplus's forward direction for a caller that will hand `z` and `out` to
+ * fpscan_scan_bwd_softplus; the output alone is kept (see fpscan_scan_fwd_saved). */
+int fpscan_scan_fwd_softplus_saved(const void* z, const float* rate, const void* tokens,
+                                   void* out, int64_t batch, int64_t dim, int64_t seqlen,
+                                   int64_t stride_b, int64_t stride_d, int dtype,
+                                   void* stream);
 
 /* Fused backward of fpscan_scan_fwd_softplus (forward direction), given its output `out`:
  * grad_tokens as fpscan_scan_bwd; grad_z = grad_gates * gate * (-rate) * sigmoid(z); and, if
