@@ -235,8 +235,8 @@ void check_input_cl(const at::Tensor& t, const char* name) {
               t.scalar_type(), " (16-byte vectors), got ", t.size(2));
 }
 
-at::Tensor fullscan_forward_cl(const at::Tensor& Ax, const at::Tensor& Bx, const at::Tensor& out,
-                               bool reverse) {
+at::Tensor run_forward_cl(const at::Tensor& Ax, const at::Tensor& Bx, const at::Tensor& out,
+                          bool reverse, bool saved) {
   check_input_cl(Ax, "Ax");
   check_input_cl(Bx, "Bx");
   check_like(Ax, Bx, "Ax", "Bx");
@@ -251,11 +251,24 @@ at::Tensor fullscan_forward_cl(const at::Tensor& Ax, const at::Tensor& Bx, const
   const int dt = dtype_code(Bx.scalar_type());
   const size_t ws_bytes = fpscan_workspace_bytes_cl(B, L, D, D, dt, FPSCAN_OP_FWD);
   at::Tensor ws = workspace(ws_bytes, Bx);
-  const int status = fpscan_scan_fwd_cl(Ax.data_ptr(), Bx.data_ptr(), out.data_ptr(), B, L, D,
-                                        L * D, D, dt, reverse ? 1 : 0,
-                                        ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, stream);
+  void* w = ws_bytes ? ws.data_ptr() : nullptr;
+  const int status =
+      saved ? fpscan_scan_fwd_cl_saved(Ax.data_ptr(), Bx.data_ptr(), out.data_ptr(), B, L, D,
+                                       L * D, D, dt, w, ws_bytes, stream)
+            : fpscan_scan_fwd_cl(Ax.data_ptr(), Bx.data_ptr(), out.data_ptr(), B, L, D, L * D, D,
+                                 dt, reverse ? 1 : 0, w, ws_bytes, stream);
   check_status(status);
   return out;
+}
+
+at::Tensor fullscan_forward_cl(const at::Tensor& Ax, const at::Tensor& Bx, const at::Tensor& out,
+                               bool reverse) {
+  return run_forward_cl(Ax, Bx, out, reverse, false);
+}
+
+at::Tensor fullscan_forward_cl_saved(const at::Tensor& Ax, const at::Tensor& Bx,
+                                     const at::Tensor& out) {
+  return run_forward_cl(Ax, Bx, out, false, true);
 }
 
 std::tuple<at::Tensor, at::Tensor> fullscan_backward_cl(const at::Tensor& gates,
@@ -452,6 +465,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fullscan_forward_cl", &fullscan_forward_cl,
         "channel-last scan of (batch, seqlen, dim) tensors along seqlen, written into out",
         pybind11::arg("Ax"), pybind11::arg("Bx"), pybind11::arg("out"), pybind11::arg("reverse"));
+  m.def("fullscan_forward_cl_saved", &fullscan_forward_cl_saved,
+        "fullscan_forward_cl for a training step (see fullscan_forward_saved)",
+        pybind11::arg("Ax"), pybind11::arg("Bx"), pybind11::arg("out"));
   m.def("fullscan_backward_cl", &fullscan_backward_cl,
         "fused backward of the channel-last forward scan: (grad_gates, grad_tokens)",
         pybind11::arg("gates"), pybind11::arg("out"), pybind11::arg("grad_out"),

@@ -14,11 +14,12 @@
 //   Each lane carries the V independent recurrences of its vector down the time axis, so
 //   there is no cross-lane scan at all: per step, y = fma(a, y, b) on V values. One wave owns
 //   one strip of one batch over a segment of time steps, with a ring of U steps in flight.
-//   When batch x strips alone cannot fill the device, the time axis is tiled instead: with
-//   enough 64-column chains, one pass over tiles of 64 columns with a look-back along time
-//   (scan_cl_tiles below, 3 N s bytes forward); otherwise segments in three launches (per-
-//   segment per-column aggregates (A, B) into the workspace, a carry pass over the segments of
-//   each column, then the segments again with their carry-in: 5 N s bytes forward).
+//   When batch x strips alone cannot fill the device, the time axis is tiled instead, one pass
+//   (3 N s bytes forward) with a look-back along time: scan_cl_blocks (a tile per 256-thread
+//   workgroup), or from 1 GiB per tensor scan_cl_tiles (a persistent grid with a ring of
+//   tiles). Where neither applies, segments in three launches (per-segment per-column
+//   aggregates (A, B) into the workspace, a carry pass over the segments of each column, then
+//   the segments again with their carry-in: 5 N s bytes forward).
 // All arithmetic is fp32; half types are widened exactly on load and rounded to nearest even
 // once on store.
 #include <hip/hip_runtime.h>
@@ -68,6 +69,10 @@ struct ClArgs {
   // forces waits to give up) and the polls before a wait gives up
   int64_t skip_publish;
   int32_t spin_limit;
+  // block path: 16-byte vectors per panel, panels per batch, row groups per tile
+  int32_t cv;
+  int32_t npan;
+  int32_t groups;
 };
 
 // Look-back waits of the tiled channel-last kernel that gave up on this device since the
@@ -836,6 +841,308 @@ scan_cl_tiles(const ClArgs a, uint64_t* __restrict__ status, const int64_t ntile
 }
 
 // ---------------------------------------------------------------------------------------
+// Block channel-last scan: one tile per 256-thread workgroup, several workgroups per CU.
+//
+// A panel is `cv` consecutive 16-byte vectors of a row; a tile is `groups` x R consecutive
+// time steps of one panel (groups = 256 / cv), a chain one batch's panel over the whole time
+// axis. Lane (group g, vector c) = thread g cv + c holds R consecutive steps of V columns.
+// The whole tile is loaded at once; then
+//   1. each lane composes its R steps serially into one map (A, B) per column -> LDS;
+//   2. thread q < cv V, one per column, composes the groups' maps into the tile's aggregate,
+//      publishes it, finds the carry from the predecessors' words (as in scan_cl_tiles:
+//      agg(k-1) o ... o agg(k-K) applied to y_end(k-K-1), always the same way), and leaves
+//      the value entering each group in LDS;
+//   3. each lane re-runs its steps from that value and stores.
+// A workgroup claims its tile when it starts (Claims: within a claim group all chains' tile 0,
+// then all chains' tile 1, ...), so a tile waits only for tiles that running workgroups hold.
+// With a single tile per chain there is nothing to wait for, and no workspace.
+//
+// Against scan_cl_tiles (one 1024-thread workgroup per CU with a ring of tiles): no start-up
+// chain of claims, no ring to fill and drain, so a call of tens of microseconds is shorter;
+// the other workgroups of the CU cover a tile's waits instead of the ring. The bound is the
+// memory system, through the launch, the claim and the look-back of a few tiles per CU.
+// Measured on MI355X, forward + backward with their status clears, scan_cl_tiles -> this
+// kernel (us): bf16 (8, 2048, 1024) 28.8 + 47.2 -> 28.1 + 38.7, (2, 2048, 1024) 15.2 + 17.7 ->
+// 11.4 + 13.2, (1, 65536, 1024) 102.3 + 145.2 -> 85.8 + 135.8, (4, 4096, 2048) 50.4 + 78.8 ->
+// 45.3 + 70.8, f16 (3, 1000, 776) 17.5 + 19.7 -> 12.1 + 13.9, fp32 (4, 4096, 1024) 49.9 + 74.9
+// -> 43.2 + 68.2. Panels of 128 bytes (cv = 8): 256-byte panels put two waves into step 2 and
+// measured 2-10 % slower, wider ones more. K = 8 aggregates: 16 take 32 registers more (and
+// spill at R = 8), 1-3 % slower; 4 lose 8 % with few chains. The forward takes R = 8 (256 steps
+// a tile; 4 measured up to 20 % slower with few chains, even otherwise), the backward R = 4,
+// or 8 below kClbFewChains, where the look-back's latency bounds it (see plan_cl_blocks).
+//
+// Cache policies (kPol): streamed; kClbSaved, the forward of a training step (gates and
+// output left in the memory-side cache, see kKeepBoth); kClbShared, rows that do not start on
+// 128-byte lines: a panel's pieces then share lines with the neighbouring panels and rows, and
+// with the nontemporal policy each piece fetches, and worse, writes back its lines by itself.
+// ---------------------------------------------------------------------------------------
+constexpr int kClbThreads = 256;
+constexpr int kClbAggs = 8;
+constexpr int kClbCv = 8;      // vectors per panel aimed at
+constexpr int kClbMaxCv = 32;  // step 2 needs a thread per column: cv V <= 256
+
+constexpr int kClbStream = 0;
+constexpr int kClbSaved = 1;
+constexpr int kClbShared = 2;
+
+template <class E, int kMode, int R, int kPol>
+__global__ void __launch_bounds__(kClbThreads, (kMode == kBwd && R == 8) ? 3 : 4)
+scan_cl_blocks(const ClArgs a, uint64_t* __restrict__ status, const int64_t ntiles) {
+  constexpr int V = E::V;
+  constexpr int K = kClbAggs;
+  constexpr int kGatePol = kPol == kClbStream ? kCacheNT : 0;
+  constexpr int kInPol = kPol == kClbShared ? 0 : kCacheNT;
+  constexpr int kOutPol = kPol == kClbStream ? kCacheNT : 0;
+  constexpr bool kReverse = kMode != kFwd;
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+  __shared__ f32x4 maps[V / 2][kClbThreads];    // plane i: columns 2i, 2i+1 of the vector
+  __shared__ f32x4 entry[V / 4][kClbThreads];   // plane j: columns 4j..4j+3
+  __shared__ int64_t claimed;
+
+  const int tid = threadIdx.x;
+  const int cv = a.cv;
+  const int ncols = cv * V;
+  const int64_t nagg = ntiles * ncols;
+  const int64_t nstatus = nagg + nagg / 2;
+  const bool chained = status != nullptr;
+  const ChainGroups cg{a.chains, a.nseg};
+  if (chained) {
+    const Rsrc st = __builtin_amdgcn_make_buffer_rsrc(
+        status, (short)0, (int)((nstatus + kStatusExtraWords) * sizeof(uint64_t)), kRsrcWord3);
+    if (tid == 0) {
+      Claims<ChainGroups> claims{
+          (uint32_t)((nstatus + kCounterStride) * sizeof(uint64_t)),
+          reinterpret_cast<const uint32_t*>(status + nstatus + kCounterStride), cg,
+          (int)(blockIdx.x % kClaimGroups)};
+      claimed = claims.next_now(st, ntiles, ntiles + 1);
+    }
+    __syncthreads();
+  }
+  const int64_t tile = chained ? (int64_t)__builtin_amdgcn_readfirstlane((int)claimed)
+                               : (int64_t)blockIdx.x;
+  if (tile >= ntiles) return;  // uniform
+
+  // the tile's claim group, chain and segment
+  int seg = 0, nch = 1;
+  int64_t chain = tile;
+  if (chained) {
+    int g = 0;
+#pragma unroll
+    for (int i = 1; i < kClaimGroups; ++i) g += tile >= cg.first(i) ? 1 : 0;
+    const int64_t c_lo = cg.chain_lo(g);
+    nch = (int)(cg.chain_lo(g + 1) - c_lo);
+    const uint32_t k = (uint32_t)(tile - c_lo * a.nseg);
+    seg = __builtin_amdgcn_readfirstlane((int)(k / (uint32_t)nch));
+    chain = c_lo + (int64_t)(k - (uint32_t)seg * (uint32_t)nch);
+  }
+  const int64_t b = __builtin_amdgcn_readfirstlane((uint32_t)chain / (uint32_t)a.npan);
+  const int pan = (int)(chain - b * a.npan);
+
+  const int L = a.seqlen;
+  const int T = a.groups * R;
+  const int p0 = seg * T;
+  const int p1 = min(p0 + T, L);
+  const int lo = kReverse ? L - p1 : p0;
+  const int hi = kReverse ? L - p0 : p1;
+  const int r0 = lo > 0 ? lo - 1 : 0;
+  const int r1 = hi < L ? hi + 1 : L;
+  const uint32_t row_bytes = (uint32_t)(a.stride_t * E::kSize);
+  const int64_t base = b * a.stride_b + (int64_t)r0 * a.stride_t;
+  const int32_t bytes = (int32_t)((uint32_t)(r1 - r0) * row_bytes);
+
+  const int g = tid / cv;
+  const int c = tid - g * cv;
+  const int col = (pan * cv + c) * V;
+  const bool active = g < a.groups && col < a.dim;
+  const int pl = p0 + g * R;  // this lane's first step, processing order
+  const uint32_t col_off = (uint32_t)col * E::kSize;
+  auto off = [&](int r) -> uint32_t {
+    const int p = pl + r;
+    const int t = kReverse ? L - 1 - p : p;
+    return active && p < p1 ? (uint32_t)(t - r0) * row_bytes + col_off : kNoOffset;
+  };
+
+  u32x4 v0[R], v1[R], v2[kMode == kBwd ? R : 1];
+  {
+    const Rsrc in0 = cl_tile_rsrc(a.in0, base, E::kSize, bytes);
+    const Rsrc in1 = cl_tile_rsrc(a.in1, base, E::kSize, bytes);
+    const Rsrc in2 = cl_tile_rsrc(kMode == kBwd ? a.in2 : a.in1, base, E::kSize, bytes);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const uint32_t o = off(r);
+      if constexpr (kMode == kBwd) {
+        // gates[t+1] (past the end: replaced by 1 below), grad_out[t], out[t-1] (before the
+        // start: 0)
+        const int t = L - 1 - (pl + r);
+        v0[r] = bld16<kGatePol>(in0, o != kNoOffset && t + 1 < L ? o + row_bytes : kNoOffset);
+        v1[r] = bld16<kInPol>(in1, o);
+        v2[r] = bld16<kInPol>(in2, o != kNoOffset && t >= 1 ? o - row_bytes : kNoOffset);
+      } else {
+        v0[r] = bld16<kGatePol>(in0, o);
+        v1[r] = bld16<kInPol>(in1, o);
+      }
+    }
+  }
+  // the chain's first step never uses its gate (the backward's is gates[L] = 1)
+  const bool first = pl == 0;
+
+  // (1) the lane's R steps
+  {
+    float A[V], B[V];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      float ga[V], xb[V];
+      E::unpack(v0[r], ga);
+      E::unpack(v1[r], xb);
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        if (r == 0) {
+          A[e] = first ? 1.0f : ga[e];
+          B[e] = xb[e];
+        } else {
+          B[e] = fmaf(ga[e], B[e], xb[e]);
+          A[e] = ga[e] * A[e];
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < V / 2; ++i)
+      maps[i][tid] = f32x4{A[2 * i], B[2 * i], A[2 * i + 1], B[2 * i + 1]};
+  }
+  lds_barrier();
+
+  // (2) one thread per column: aggregate, look-back, the value entering each group
+  if (tid < ncols) {
+    const int h = tid & 1;
+    const int qi = (tid >> 1) / cv;
+    const int qc = (tid >> 1) - qi * cv;
+    const f32x2* col_maps = reinterpret_cast<const f32x2*>(&maps[qi][qc]) + h;  // stride 2 cv
+    float carry = 0.0f;
+    if (chained) {
+      float A = 1.0f, B = 0.0f;
+#pragma unroll 4
+      for (int i = 0; i < a.groups; ++i) {
+        const f32x2 m = col_maps[2 * i * cv];
+        B = fmaf(m.x, B, m.y);
+        A = m.x * A;
+      }
+      const Rsrc st = __builtin_amdgcn_make_buffer_rsrc(
+          status, (short)0, (int)((nstatus + kStatusExtraWords) * sizeof(uint64_t)), kRsrcWord3);
+      const uint32_t ends_off = (uint32_t)(nagg * sizeof(uint64_t));
+      if (tile != a.skip_publish && seg + 1 < a.nseg)
+        status_store(st, (uint32_t)((tile * ncols + tid) * sizeof(uint64_t)), pack_map(A, B));
+      if (seg > 0) {
+        const int na = min(seg, K);
+        uint64_t words[K];
+        uint32_t end = 0;
+#pragma unroll
+        for (int j = 0; j < K; ++j)
+          words[j] = status_load(
+              st, j < na ? (uint32_t)(((tile - (int64_t)(j + 1) * nch) * ncols + tid) *
+                                      sizeof(uint64_t))
+                         : kNoOffset);
+        const uint32_t end_at =
+            ends_off + (uint32_t)(((tile - (int64_t)(K + 1) * nch) * ncols + tid) *
+                                  sizeof(uint32_t));
+        end = end_load(st, seg > K ? end_at : kNoOffset);
+        if (__builtin_amdgcn_ballot_w64(agg_missing(words, na) ||
+                                        (seg > K && end == kEndNotPublished)) != 0) {
+          const bool overran = __hip_atomic_load(status + nstatus, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT) != 0;
+          for (int it = overran ? a.spin_limit : 0;; ++it) {
+            __builtin_amdgcn_s_sleep(1);
+#pragma unroll
+            for (int j = 0; j < K; ++j)
+              if (j < na && words[j] == kNotPublished)
+                words[j] = __hip_atomic_load(
+                    status + (tile - (int64_t)(j + 1) * nch) * ncols + tid, __ATOMIC_RELAXED,
+                    __HIP_MEMORY_SCOPE_AGENT);
+            if (seg > K && end == kEndNotPublished)
+              end = __hip_atomic_load(reinterpret_cast<const uint32_t*>(status) + end_at / 4,
+                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (__builtin_amdgcn_ballot_w64(agg_missing(words, na) ||
+                                            (seg > K && end == kEndNotPublished)) == 0)
+              break;
+            if (it >= a.spin_limit) {
+              if ((tid & 63) == 0) {
+                __hip_atomic_fetch_add(status + nstatus, 1ull, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_fetch_add(&g_cl_overruns, 1ull, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+              }
+              break;
+            }
+          }
+          // only after an overrun: what is still missing becomes NaN, not plausible
+#pragma unroll
+          for (int j = 0; j < K; ++j)
+            words[j] = words[j] == kNotPublished ? kPoisonMap : words[j];
+          end = end == kEndNotPublished ? kPoisonValue : end;
+        }
+        carry = seg > K ? __uint_as_float(end) : 0.0f;
+#pragma unroll
+        for (int j = K - 1; j >= 0; --j)
+          if (j < na)
+            carry = fmaf(__uint_as_float((uint32_t)words[j]), carry,
+                         __uint_as_float((uint32_t)(words[j] >> 32)));
+      }
+      if (seg + K + 1 < a.nseg)
+        end_store(st, ends_off + (uint32_t)((tile * ncols + tid) * sizeof(uint32_t)),
+                  canonical_bits(fmaf(A, carry, B)));
+    }
+    const int e = 2 * qi + h;
+    float* enter = reinterpret_cast<float*>(&entry[e / 4][qc]) + e % 4;  // stride 4 cv
+#pragma unroll 4
+    for (int i = 0; i < a.groups; ++i) {
+      enter[4 * i * cv] = carry;
+      const f32x2 m = col_maps[2 * i * cv];
+      carry = fmaf(m.x, carry, m.y);
+    }
+  }
+  lds_barrier();
+
+  // (3) re-run the steps from the value entering the lane's group; the operands are unpacked
+  // again (left to the compiler, their fp32 forms would be held across both barriers)
+  {
+    float y[V];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      asm volatile("" : "+v"(v0[r]), "+v"(v1[r]));
+      if constexpr (kMode == kBwd) asm volatile("" : "+v"(v2[r]));
+    }
+#pragma unroll
+    for (int j = 0; j < V / 4; ++j) {
+      const f32x4 q = entry[j][tid];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[4 * j + e] = q[e];
+    }
+    const Rsrc out0 = cl_tile_rsrc(a.out0, base, E::kSize, bytes);
+    const Rsrc out1 = cl_tile_rsrc(kMode == kBwd ? a.out1 : a.out0, base, E::kSize, bytes);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      float ga[V], xb[V];
+      E::unpack(v0[r], ga);
+      E::unpack(v1[r], xb);
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        const float al = r == 0 && first ? 1.0f : ga[e];
+        y[e] = fmaf(al, y[e], xb[e]);
+      }
+      const uint32_t o = off(r);
+      bst16<kOutPol>(out0, o, E::pack(y));
+      if constexpr (kMode == kBwd) {
+        float yp[V], gg[V];
+        E::unpack(v2[r], yp);
+#pragma unroll
+        for (int e = 0; e < V; ++e) gg[e] = y[e] * yp[e];
+        bst16<kOutPol>(out1, o, E::pack(gg));
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------------------
 // One wave (one strip task) per block: blocks of four waves put each four tasks on one CU, so
@@ -985,6 +1292,17 @@ int cl_resident_blocks(const void* kernel, int slot, int threads) {
   return n;
 }
 
+// Clears the status words and counters of a look-back launch.
+int clear_cl_status(uint64_t* status, int64_t nstatus, hipStream_t stream) {
+  const int64_t nwords = nstatus + kStatusExtraWords;
+  const int64_t blocks = (nwords + 255) / 256 < 2048 ? (nwords + 255) / 256 : 2048;
+  void* args[] = {&status, &nstatus};
+  return hipLaunchKernel(reinterpret_cast<const void*>(&clear_status), dim3((unsigned)blocks),
+                         dim3(256), args, 0, stream) == hipSuccess
+             ? FPSCAN_OK
+             : FPSCAN_ERR_LAUNCH;
+}
+
 // Clears the status words and counters, then the persistent grid. -1 when the occupancy query
 // fails (the caller then takes another path).
 template <class E, int kMode>
@@ -1017,13 +1335,8 @@ int run_cl_tiled(ClArgs a, const ClTilePlan& plan, void* workspace, hipStream_t 
   if (resident <= 0) return -1;
   uint64_t* status = static_cast<uint64_t*>(workspace);
   int64_t ntiles = plan.ntiles;
-  int64_t nstatus = cl_status_words(ntiles);
-  const int64_t nwords = nstatus + kStatusExtraWords;
-  const int64_t clear_blocks = (nwords + 255) / 256 < 2048 ? (nwords + 255) / 256 : 2048;
-  void* cargs[] = {&status, &nstatus};
-  if (hipLaunchKernel(reinterpret_cast<const void*>(&clear_status), dim3((unsigned)clear_blocks),
-                      dim3(256), cargs, 0, stream) != hipSuccess)
-    return FPSCAN_ERR_LAUNCH;
+  const int cst = clear_cl_status(status, cl_status_words(ntiles), stream);
+  if (cst != FPSCAN_OK) return cst;
   int64_t grid = resident;
   if (grid > ntiles) grid = ntiles;
   a.chains = plan.chains;
@@ -1039,8 +1352,107 @@ int run_cl_tiled(ClArgs a, const ClTilePlan& plan, void* workspace, hipStream_t 
   return err == hipSuccess ? FPSCAN_OK : FPSCAN_ERR_LAUNCH;
 }
 
+// Block path (scan_cl_blocks): tile geometry, workspace, and where it is taken.
+struct ClBlockPlan {
+  bool use;
+  bool shared;  // rows off the 128-byte lines
+  int cv, npan, groups, r;
+  int64_t chains, nseg, ntiles;
+  size_t bytes;  // workspace: a status word and an end value per tile and column, overrun word
+                 // and claim counters; 0 with one tile per chain
+};
+
+// The backward takes R = 8 below this many chains. Measured on MI355X, R = 4 against 8 (us):
+// 16 chains, bf16 (1, 65536, 1024) 143.0 / 135.8, 39 chains, f16 (3, 1000, 776) 17.3 / 13.9; 32
+// chains, bf16 (2, 2048, 1024) 13.2 / 13.5; 128 chains, bf16 (8, 2048, 1024) 38.7 / 41.0 and (4,
+// 4096, 2048) 70.8 / 71.2, 256 chains, bf16 (16, 1024, 1024) 37.2 / 38.6.
+constexpr int64_t kClbFewChains = 48;
+// Rows on 128-byte lines go to scan_cl_tiles from this size per tensor: at 512 MiB, bf16 (4,
+// 65536, 1024), this kernel takes 290 + 480 us against 312 + 480, at 1 GiB, (8, 65536, 1024),
+// 572 + 965 against 567 + 925.
+constexpr int64_t kClbMaxBytes = 1ll << 30;
+// The largest tensor whose gates and output the forward of a training step keeps (as for rows).
+constexpr int64_t kClKeepMaxBytes = 128ll << 20;
+
+// Taken in the automatic mode where one pass per strip lacks strips, whatever the size when
+// the rows are off the lines, else below kClbMaxBytes. Off the lines (measured on MI355X,
+// forward + backward, scan_cl_tiles -> this kernel, us): f16 (45, 12181, 240) 239 + 451 -> 193 +
+// 294, bf16 (56, 10271, 360) 512 + 906 -> 323 + 552, (8, 16384, 776) 178 + 360 -> 144 + 249, (10,
+// 32768, 1032) 636 + 1301 -> 479 + 928. There also with enough strips, if a chain has several
+// tiles: bf16 (64, 512, 4104) one pass 204 + 364 -> 203 + 356; on the lines the one pass is the
+// faster one (fp32 (64, 256, 4096) 138 + 243 against 158 + 261).
+ClBlockPlan plan_cl_blocks(int64_t batch, int64_t seqlen, int64_t dim, int64_t stride_t, int size,
+                           int tiling, bool bwd) {
+  ClBlockPlan t{};
+  if (tiling != 0 || batch <= 0 || seqlen <= 0 || dim <= 0) return t;
+  const int vec = cl_vec(size);
+  const int64_t nv = (dim + vec - 1) / vec;
+  t.shared = (stride_t * size) % 128 != 0;
+  // narrow rows off the lines: a panel holds the whole row, so that tiles are contiguous (f16
+  // (45, 12181, 240) backward 350 -> 294 us); otherwise panels of up to kClbCv vectors
+  t.npan = (int)(t.shared && nv <= kClbMaxCv ? 1 : (nv + kClbCv - 1) / kClbCv);
+  t.cv = (int)((nv + t.npan - 1) / t.npan);
+  t.groups = kClbThreads / t.cv;
+  t.chains = batch * t.npan;
+  t.r = bwd && !t.shared && t.chains >= kClbFewChains ? 4 : 8;
+  const int64_t steps = (int64_t)t.groups * t.r;
+  t.nseg = (seqlen + steps - 1) / steps;
+  t.ntiles = t.chains * t.nseg;
+  const int64_t words = t.ntiles * t.cv * vec * 3 / 2 + kStatusExtraWords;
+  if (t.ntiles > INT32_MAX / kClbThreads || words * (int64_t)sizeof(uint64_t) > INT32_MAX ||
+      (steps + 2) * stride_t * size > INT32_MAX)
+    return t;
+  const bool enough_strips = batch * ((nv + 63) / 64) >= kClMinTasks;
+  if (t.shared ? enough_strips && t.nseg < 2
+               : enough_strips || batch * seqlen * dim * size >= kClbMaxBytes)
+    return t;
+  t.use = true;
+  t.bytes = t.nseg > 1 ? (size_t)words * sizeof(uint64_t) : 0;
+  return t;
+}
+
+template <class E, int kMode, int R>
+const void* cl_blocks_kernel(bool shared, bool saved) {
+  if (shared) return reinterpret_cast<const void*>(&scan_cl_blocks<E, kMode, R, kClbShared>);
+  if constexpr (kMode == kFwd) {
+    if (saved) return reinterpret_cast<const void*>(&scan_cl_blocks<E, kMode, R, kClbSaved>);
+  }
+  return reinterpret_cast<const void*>(&scan_cl_blocks<E, kMode, R, kClbStream>);
+}
+
 template <class E, int kMode>
-int run_cl(ClArgs a, void* workspace, size_t ws_bytes, hipStream_t stream) {
+int run_cl_blocks(ClArgs a, const ClBlockPlan& plan, bool saved, void* workspace,
+                  hipStream_t stream) {
+  const void* kernel = cl_blocks_kernel<E, kMode, 8>(plan.shared, saved);
+  if constexpr (kMode == kBwd) {
+    if (plan.r == 4) kernel = cl_blocks_kernel<E, kMode, 4>(plan.shared, saved);
+  }
+  uint64_t* status = plan.nseg > 1 ? static_cast<uint64_t*>(workspace) : nullptr;
+  int64_t ntiles = plan.ntiles;
+  if (status != nullptr) {
+    const int st = clear_cl_status(status, ntiles * plan.cv * E::V * 3 / 2, stream);
+    if (st != FPSCAN_OK) return st;
+  }
+  a.cv = plan.cv;
+  a.npan = plan.npan;
+  a.groups = plan.groups;
+  a.chains = plan.chains;
+  a.nseg = (int32_t)plan.nseg;
+  a.ws = nullptr;
+  a.skip_publish = fpscan_detail::hook_skip_publish();
+  a.spin_limit = fpscan_detail::hook_spin_limit();
+  void* kargs[] = {&a, &status, &ntiles};
+  const hipError_t err =
+      hipLaunchKernel(kernel, dim3((unsigned)ntiles), dim3(kClbThreads), kargs, 0, stream);
+  return err == hipSuccess ? FPSCAN_OK : FPSCAN_ERR_LAUNCH;
+}
+
+template <class E, int kMode>
+int run_cl(ClArgs a, bool saved, void* workspace, size_t ws_bytes, hipStream_t stream) {
+  const ClBlockPlan blocks = plan_cl_blocks(a.batch, a.seqlen, a.dim, a.stride_t, E::kSize,
+                                            fpscan_detail::tiling_mode(), kMode == kBwd);
+  if (blocks.use && (blocks.bytes == 0 || (workspace != nullptr && ws_bytes >= blocks.bytes)))
+    return run_cl_blocks<E, kMode>(a, blocks, saved, workspace, stream);
   const ClTilePlan tiles = plan_cl_tiles(a.batch, a.seqlen, a.dim, a.stride_t, E::kSize,
                                          fpscan_detail::tiling_mode());
   if (tiles.use && workspace != nullptr && ws_bytes >= tiles.bytes) {
@@ -1073,11 +1485,12 @@ int run_cl(ClArgs a, void* workspace, size_t ws_bytes, hipStream_t stream) {
 }
 
 template <int kMode>
-int dispatch_cl(int dtype, const ClArgs& a, void* ws, size_t ws_bytes, hipStream_t stream) {
+int dispatch_cl(int dtype, const ClArgs& a, bool saved, void* ws, size_t ws_bytes,
+                hipStream_t stream) {
   switch (dtype) {
-    case FPSCAN_DTYPE_F32: return run_cl<F32, kMode>(a, ws, ws_bytes, stream);
-    case FPSCAN_DTYPE_F16: return run_cl<F16, kMode>(a, ws, ws_bytes, stream);
-    case FPSCAN_DTYPE_BF16: return run_cl<BF16, kMode>(a, ws, ws_bytes, stream);
+    case FPSCAN_DTYPE_F32: return run_cl<F32, kMode>(a, saved, ws, ws_bytes, stream);
+    case FPSCAN_DTYPE_F16: return run_cl<F16, kMode>(a, saved, ws, ws_bytes, stream);
+    case FPSCAN_DTYPE_BF16: return run_cl<BF16, kMode>(a, saved, ws, ws_bytes, stream);
     default: return FPSCAN_ERR_DTYPE;
   }
 }
@@ -1143,10 +1556,10 @@ int cl_overruns(unsigned long long* count) {
 
 extern "C" {
 
-int fpscan_scan_fwd_cl(const void* gates, const void* tokens, void* out, int64_t batch,
-                       int64_t seqlen, int64_t dim, int64_t stride_b, int64_t stride_t,
-                       int dtype, int reverse, void* workspace, size_t workspace_bytes,
-                       void* stream) {
+static int forward_cl(const void* gates, const void* tokens, void* out, int64_t batch,
+                      int64_t seqlen, int64_t dim, int64_t stride_b, int64_t stride_t, int dtype,
+                      bool reverse, bool saved, void* workspace, size_t workspace_bytes,
+                      void* stream) {
   ClArgs a{};
   const void* ptrs[] = {gates, tokens, out};
   const int st = validate_cl(batch, seqlen, dim, stride_b, stride_t, dtype, ptrs, 3, a);
@@ -1158,8 +1571,29 @@ int fpscan_scan_fwd_cl(const void* gates, const void* tokens, void* out, int64_t
   a.out0 = out;
   a.out1 = nullptr;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return reverse ? dispatch_cl<kRev>(dtype, a, workspace, workspace_bytes, s)
-                 : dispatch_cl<kFwd>(dtype, a, workspace, workspace_bytes, s);
+  return reverse ? dispatch_cl<kRev>(dtype, a, false, workspace, workspace_bytes, s)
+                 : dispatch_cl<kFwd>(dtype, a, saved, workspace, workspace_bytes, s);
+}
+
+int fpscan_scan_fwd_cl(const void* gates, const void* tokens, void* out, int64_t batch,
+                       int64_t seqlen, int64_t dim, int64_t stride_b, int64_t stride_t,
+                       int dtype, int reverse, void* workspace, size_t workspace_bytes,
+                       void* stream) {
+  return forward_cl(gates, tokens, out, batch, seqlen, dim, stride_b, stride_t, dtype,
+                    reverse != 0, false, workspace, workspace_bytes, stream);
+}
+
+int fpscan_scan_fwd_cl_saved(const void* gates, const void* tokens, void* out, int64_t batch,
+                             int64_t seqlen, int64_t dim, int64_t stride_b, int64_t stride_t,
+                             int dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  // kept only while the gates and the output fit the memory-side cache together
+  const int size = cl_itemsize(dtype);
+  int64_t elems = 0;
+  const bool fits = !__builtin_mul_overflow(batch, seqlen, &elems) &&
+                    !__builtin_mul_overflow(elems, dim, &elems) && size > 0 &&
+                    elems <= kClKeepMaxBytes / size;
+  return forward_cl(gates, tokens, out, batch, seqlen, dim, stride_b, stride_t, dtype, false, fits,
+                    workspace, workspace_bytes, stream);
 }
 
 int fpscan_scan_bwd_cl(const void* gates, const void* out, const void* grad_out,
@@ -1176,7 +1610,8 @@ int fpscan_scan_bwd_cl(const void* gates, const void* out, const void* grad_out,
   a.in2 = out;
   a.out0 = grad_tokens;
   a.out1 = grad_gates;
-  return dispatch_cl<kBwd>(dtype, a, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+  return dispatch_cl<kBwd>(dtype, a, false, workspace, workspace_bytes,
+                           static_cast<hipStream_t>(stream));
 }
 
 size_t fpscan_workspace_bytes_cl(int64_t batch, int64_t seqlen, int64_t dim, int64_t stride_t,
@@ -1189,10 +1624,15 @@ size_t fpscan_workspace_bytes_cl(int64_t batch, int64_t seqlen, int64_t dim, int
   if (__builtin_mul_overflow(batch, seqlen, &steps) ||
       __builtin_mul_overflow(steps, stride_t, &elems) || elems > ((int64_t)1 << 48) / size)
     return 0;  // no call of this size passes validation
+  const ClBlockPlan blocks = plan_cl_blocks(batch, seqlen, dim, stride_t, size,
+                                            fpscan_detail::tiling_mode(), op == FPSCAN_OP_BWD);
   const ClTilePlan tiles =
       plan_cl_tiles(batch, seqlen, dim, stride_t, size, fpscan_detail::tiling_mode());
-  if (tiles.use) return tiles.bytes;
-  return plan_cl(batch, seqlen, dim, stride_t, size).bytes;
+  // the block path's words fit into the tiled path's almost always (off the lines its tiles
+  // can be shorter); the larger of the two serves both
+  const size_t other =
+      tiles.use ? tiles.bytes : plan_cl(batch, seqlen, dim, stride_t, size).bytes;
+  return blocks.use && blocks.bytes > other ? blocks.bytes : other;
 }
 
 }  // extern "C"

@@ -159,7 +159,8 @@ class PScanChannelLast(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, gates: torch.Tensor, tokens: torch.Tensor) -> torch.Tensor:
-        out = scan_forward_channel_last(gates, tokens)
+        out = torch.empty_like(tokens)
+        _load_extension().fullscan_forward_cl_saved(gates, tokens, out)
         ctx.save_for_backward(gates, out)
         return out
 

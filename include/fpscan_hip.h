@@ -166,6 +166,13 @@ int fpscan_scan_fwd_cl(const void* gates, const void* tokens, void* out,
                        int dtype, int reverse,
                        void* workspace, size_t workspace_bytes, void* stream);
 
+/* fpscan_scan_fwd_cl's forward direction for a caller that will hand `gates` and `out` to
+ * fpscan_scan_bwd_cl (see fpscan_scan_fwd_saved): the same results and workspace. */
+int fpscan_scan_fwd_cl_saved(const void* gates, const void* tokens, void* out,
+                             int64_t batch, int64_t seqlen, int64_t dim,
+                             int64_t stride_b, int64_t stride_t, int dtype,
+                             void* workspace, size_t workspace_bytes, void* stream);
+
 /* Fused backward of fpscan_scan_fwd_cl (forward direction), given its output `out`:
  *   grad_tokens[b,t,d] = grad_out[b,t,d] + gates[b,t+1,d] * grad_tokens[b,t+1,d]  (gates[b,L,d] = 1)
  *   grad_gates[b,t,d]  = grad_tokens[b,t,d] * out[b,t-1,d]                      (out[b,-1,d] = 0)
@@ -178,8 +185,9 @@ int fpscan_scan_bwd_cl(const void* gates, const void* out, const void* grad_out,
                        int dtype,
                        void* workspace, size_t workspace_bytes, void* stream);
 
-/* Workspace, in bytes, for the tiled or segmented channel-last path this problem takes (0: one
- * pass per strip); it depends on fpscan_set_tiling's setting. */
+/* Workspace, in bytes, for the path with a look-back (tiles or blocks) or the segments that
+ * this problem takes (0: one pass per strip); it depends on fpscan_set_tiling's setting and can
+ * differ between the operations. */
 size_t fpscan_workspace_bytes_cl(int64_t batch, int64_t seqlen, int64_t dim, int64_t stride_t,
                                  int dtype, int op);
 

@@ -1,0 +1,156 @@
+"""GPU tests of the block channel-last scan, which the automatic choice takes where one pass per
+strip lacks strips: one tile of 256 threads per workgroup, panels of up to 8 (rows off the
+128-byte lines: up to 32) 16-byte vectors, 4 or 8 steps per lane, a look-back of depth 8.
+
+Against the oracle on integer data bit for bit (gates 0 or 1, every partial result exact) and
+on random data, at the edges of tiles, panels and look-back depth; its workspace bounds,
+padded strides, in-place use, determinism, and a look-back wait that gives up.
+"""
+import pytest
+import torch
+
+import fpscan_amd
+import oracle
+from fpscan_amd import ops
+from scan_helpers import DEVICE, DTYPES, bits_equal, check
+from test_scan_cl_tiled_gpu import _CODE, cl_inputs, lib  # noqa: F401  (fixture)
+
+pytestmark = [
+    pytest.mark.gpu,
+    pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device (MI355X)"),
+]
+
+# (batch, seqlen, 16-byte vectors per row): on the lines, 8 vectors = 32 groups: tiles of 256
+# steps (8 per lane), of 128 in the backward from 48 chains; one tile exactly, one step less
+# and more; 11 tiles (an end value two look-backs back); off the lines, whole rows as panels
+# (1, 2, 9, 31 vectors: 256, 128, 28, 8 groups) and split ones (33 -> 5 panels of 7); 2 batches of
+# 24 panels: the backward's shorter tiles
+SHAPES = [(1, 255, 8), (2, 256, 8), (1, 257, 8), (1, 2600, 8), (3, 300, 16), (2, 2049, 1),
+          (1, 4500, 2), (2, 3000, 9), (3, 700, 31), (1, 1000, 33), (2, 1300, 24 * 8), (5, 1, 40),
+          (2, 127, 24 * 8), (2, 129, 24 * 8)]
+
+
+def _shape(shape, dtype):
+    B, L, nv = shape
+    return B, L, nv * (16 // torch.empty((), dtype=dtype).element_size())
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_exact_on_integer_data(dtype, shape):
+    shape = _shape(shape, dtype)
+    gen = torch.Generator().manual_seed(sum(shape))
+    g = (torch.randint(0, 6, shape, generator=gen) > 0).to(dtype)
+    x = torch.randint(-2, 3, shape, generator=gen).to(dtype)
+    go = torch.randint(-2, 3, shape, generator=gen).to(dtype)
+    gd, xd, god = g.to(DEVICE), x.to(DEVICE), go.to(DEVICE)
+    ext = ops._load_extension()
+    for rev in (False, True):
+        want = torch.from_numpy(oracle.scan_f64_channel_last(g, x, rev))
+        assert want.abs().max() < 256  # exact in every dtype
+        assert bits_equal(fpscan_amd.scan_forward_channel_last(gd, xd, rev).cpu(), want.to(dtype))
+        y = xd.clone()
+        fpscan_amd.scan_forward_channel_last(gd, y, rev, out=y)
+        assert bits_equal(y.cpu(), want.to(dtype)), "in place"
+    want = torch.from_numpy(oracle.scan_f64_channel_last(g, x, False)).to(dtype)
+    out = torch.full_like(xd, float("nan"))
+    ext.fullscan_forward_cl_saved(gd, xd, out)
+    assert bits_equal(out.cpu(), want), "the forward of a training step"
+    gg_ref, gx_ref = oracle.scan_bwd_f64_channel_last(g, want, go)
+    assert abs(gx_ref).max() < 256 and (dtype != torch.bfloat16 or abs(gg_ref).max() < 2 ** 16)
+    gg, gx = fpscan_amd.scan_backward_channel_last(gd, out, god)
+    assert bits_equal(gx.cpu(), torch.from_numpy(gx_ref).to(dtype))
+    # one rounding of an exact fp32 product
+    assert bits_equal(gg.cpu(), torch.from_numpy(gg_ref).to(dtype))
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("shape", [(1, 20000, 8), (2, 5000, 33), (4, 2500, 96)], ids=str)
+def test_matches_oracle_is_deterministic_and_mirrored(dtype, shape):
+    g, x = cl_inputs(*_shape(shape, dtype), dtype, seed=7)
+    go = torch.randn(g.shape, generator=torch.Generator().manual_seed(5)).to(dtype)
+    gd, xd = g.to(DEVICE), x.to(DEVICE)
+    y = fpscan_amd.scan_forward_channel_last(gd, xd)
+    check(y, oracle.scan_f64_channel_last(g, x), dtype, f"blocks {shape}")
+    for _ in range(3):
+        assert bits_equal(fpscan_amd.scan_forward_channel_last(gd, xd), y)
+    mirrored = fpscan_amd.scan_forward_channel_last(gd.flip(1), xd.flip(1), reverse=True).flip(1)
+    assert bits_equal(mirrored, y)
+    gg, gx = fpscan_amd.scan_backward_channel_last(gd, y, go.to(DEVICE))
+    gg_ref, gx_ref = oracle.scan_bwd_f64_channel_last(g, y.cpu(), go)
+    check(gx, gx_ref, dtype, "grad_tokens")
+    check(gg, gg_ref, dtype, "grad_gates")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("nv,pad", [(8, 8), (9, 4), (40, 3)], ids=str)
+def test_padded_strides_and_workspace_bounds(lib, dtype, nv, pad):  # noqa: F811
+    """Rows inside a wider buffer, on and off the lines, with the workspace between guards."""
+    B, L, D = _shape((2, 2700, nv), dtype)
+    vec = D // nv
+    st, code = D + pad * vec, _CODE[dtype]
+    sb = L * st
+    g, x = cl_inputs(B, L, D, dtype, seed=4)
+    go = torch.randn(B, L, D, generator=torch.Generator().manual_seed(2)).to(dtype)
+
+    def embed(t):
+        buf = torch.full((B, L, st), -3.0, dtype=dtype, device=DEVICE)
+        buf[:, :, :D] = t.to(DEVICE)
+        return buf
+
+    def ws(op):
+        n = lib.fpscan_workspace_bytes_cl(B, L, D, st, code, op)
+        buf = torch.full((n + 512,), 0xA5, dtype=torch.uint8, device=DEVICE)
+        return buf, buf.data_ptr() + 256, n
+
+    gb, xb, gob = embed(g), embed(x), embed(go)
+    outb, ggb, gxb = (embed(torch.zeros_like(x)) for _ in range(3))
+    stream = torch.cuda.current_stream().cuda_stream
+    w0, p0, n0 = ws(0)
+    w1, p1, n1 = ws(1)
+    assert lib.fpscan_scan_fwd_cl(gb.data_ptr(), xb.data_ptr(), outb.data_ptr(), B, L, D, sb, st,
+                                  code, 0, p0, n0, stream) == 0
+    assert lib.fpscan_scan_bwd_cl(gb.data_ptr(), outb.data_ptr(), gob.data_ptr(), ggb.data_ptr(),
+                                  gxb.data_ptr(), B, L, D, sb, st, code, p1, n1, stream) == 0
+    torch.cuda.synchronize()
+    for w, n in ((w0, n0), (w1, n1)):
+        assert (w[:256] == 0xA5).all() and (w[256 + n:] == 0xA5).all(), "workspace overrun"
+    out = outb[:, :, :D].cpu()
+    check(out, oracle.scan_f64_channel_last(g, x), dtype, "strided fwd")
+    gg_ref, gx_ref = oracle.scan_bwd_f64_channel_last(g, out, go)
+    check(gxb[:, :, :D].cpu(), gx_ref, dtype, "strided grad_tokens")
+    check(ggb[:, :, :D].cpu(), gg_ref, dtype, "strided grad_gates")
+    for buf in (outb, ggb, gxb):
+        assert (buf[:, :, D:] == -3.0).all(), "padding was written"
+
+
+@pytest.mark.parametrize("op", ["fwd", "rev", "bwd"])
+def test_overrun_poisons_and_is_counted(op):
+    """One chain of 12 tiles of 256 steps; tile 1 never publishes, so tiles 2..9, which compose
+    its aggregate, are NaN, tiles 0 and 1 are right, and no value is anything else."""
+    L, steps = 12 * 256, 256
+    gen = torch.Generator().manual_seed(3)
+    g = (0.9 + 0.1 * torch.rand(1, L, 32, generator=gen)).to(DEVICE)
+    x, go = (torch.randn(1, L, 32, generator=gen).to(DEVICE) for _ in range(2))
+    y = fpscan_amd.scan_forward_channel_last(g, x)
+
+    def run():
+        if op == "bwd":
+            return list(fpscan_amd.scan_backward_channel_last(g, y, go))
+        return [fpscan_amd.scan_forward_channel_last(g, x, op == "rev")]
+
+    want, before = run(), fpscan_amd.lookback_overruns()
+    ops.set_lookback_test_hook(1, 64)
+    try:
+        got = run()
+        torch.cuda.synchronize()
+    finally:
+        ops.set_lookback_test_hook()
+    assert fpscan_amd.lookback_overruns() > before
+    for a, b in zip(got, want):
+        if op != "fwd":
+            a, b = a.flip(1), b.flip(1)
+        assert bits_equal(a[:, :2 * steps], b[:, :2 * steps])
+        assert torch.isnan(a[:, 2 * steps:10 * steps]).all()
+        nan = torch.isnan(a)
+        assert bits_equal(a[~nan], b[~nan])
