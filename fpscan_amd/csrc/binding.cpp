@@ -302,6 +302,31 @@ std::tuple<at::Tensor, at::Tensor> fullscan_backward_cl(const at::Tensor& gates,
   return {grad_gates, grad_tokens};
 }
 
+// The channel-last scan as an autograd function in C++ (see PScanFunction).
+struct PScanClFunction : public torch::autograd::Function<PScanClFunction> {
+  static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& gates,
+                            const at::Tensor& tokens) {
+    at::Tensor out = at::empty_like(tokens);
+    run_forward_cl(gates, tokens, out, false, gates.requires_grad() || tokens.requires_grad());
+    ctx->save_for_backward({gates, out});
+    return out;
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const at::Tensor& gates = saved[0];
+    const at::Tensor& out = saved[1];
+    at::Tensor grad_gates = at::empty_like(gates);
+    at::Tensor grad_tokens = at::empty_like(gates);
+    fullscan_backward_cl(gates, out, grads[0].contiguous(), grad_gates, grad_tokens);
+    return {grad_gates, grad_tokens};
+  }
+};
+
+at::Tensor pscan_cl(const at::Tensor& gates, const at::Tensor& tokens) {
+  return PScanClFunction::apply(gates, tokens);
+}
+
 // ---- dimwise_forward: csrc/main.cpp:10, csrc/dimwise/dimwise.h:27-42 (CHECK_INPUT on all
 // five tensors, same messages), in place into Bx, returns nothing. Added checks: one dtype
 // for all five (the reference reinterprets Bh/Wq/Wk as Ax's type), the shapes of Ax, Bh,
@@ -429,6 +454,50 @@ void fullscan_backward_softplus(const at::Tensor& z, const at::Tensor& rate,
   check_status(status);
 }
 
+// The whole backward of the softplus-gate scan: (grad_z, grad_rate, grad_tokens), with grad_rate
+// the sum of the per-row partials over the batch (fp32, rate's shape).
+std::tuple<at::Tensor, at::Tensor, at::Tensor> softplus_gradients(const at::Tensor& z,
+                                                                  const at::Tensor& rate,
+                                                                  const at::Tensor& out,
+                                                                  const at::Tensor& grad_out) {
+  check_input(z, "z");
+  at::Tensor grad_z = at::empty_like(z);
+  at::Tensor grad_tokens = at::empty_like(z);
+  const int64_t B = z.size(0), D = z.size(1);
+  at::Tensor rows = at::empty({B * D}, z.options().dtype(at::kFloat));
+  fullscan_backward_softplus(z, rate, out, grad_out, grad_z, grad_tokens, rows);
+  if (B == 1) return {grad_z, rows.view(rate.sizes()), grad_tokens};
+  if (B == 0 || D == 0) return {grad_z, at::zeros_like(rate), grad_tokens};
+  at::Tensor grad_rate = at::empty_like(rate);
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(z.device());
+  check_status(fpscan_sum_rate_rows(rows.data_ptr<float>(), grad_rate.data_ptr<float>(), B, D,
+                                    launch_stream(z)));
+  return {grad_z, grad_rate, grad_tokens};
+}
+
+// The softplus-gate scan as an autograd function in C++ (see PScanFunction).
+struct PScanSoftplusFunction : public torch::autograd::Function<PScanSoftplusFunction> {
+  static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& z,
+                            const at::Tensor& rate, const at::Tensor& tokens) {
+    at::Tensor out = at::empty_like(tokens);
+    run_forward_softplus(z, rate, tokens, out, false,
+                         z.requires_grad() || rate.requires_grad() || tokens.requires_grad());
+    ctx->save_for_backward({z, rate, out});
+    return out;
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    auto [grad_z, grad_rate, grad_tokens] =
+        softplus_gradients(saved[0], saved[1], saved[2], grads[0].contiguous());
+    return {grad_z, grad_rate, grad_tokens};
+  }
+};
+
+at::Tensor pscan_softplus(const at::Tensor& z, const at::Tensor& rate, const at::Tensor& tokens) {
+  return PScanSoftplusFunction::apply(z, rate, tokens);
+}
+
 // Look-back waits that gave up on the tensors' device since the library was loaded (waits for
 // the device first).
 uint64_t lookback_overruns(int64_t device) {
@@ -468,6 +537,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fullscan_forward_cl_saved", &fullscan_forward_cl_saved,
         "fullscan_forward_cl for a training step (see fullscan_forward_saved)",
         pybind11::arg("Ax"), pybind11::arg("Bx"), pybind11::arg("out"));
+  m.def("pscan_cl", &pscan_cl, "differentiable channel-last scan (see pscan)",
+        pybind11::arg("gates"), pybind11::arg("tokens"));
   m.def("fullscan_backward_cl", &fullscan_backward_cl,
         "fused backward of the channel-last forward scan: (grad_gates, grad_tokens)",
         pybind11::arg("gates"), pybind11::arg("out"), pybind11::arg("grad_out"),
@@ -479,6 +550,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fullscan_forward_softplus_saved", &fullscan_forward_softplus_saved,
         "fullscan_forward_softplus for a training step (see fullscan_forward_saved)",
         pybind11::arg("z"), pybind11::arg("rate"), pybind11::arg("tokens"), pybind11::arg("out"));
+  m.def("pscan_softplus", &pscan_softplus, "differentiable softplus-gate scan (see pscan)",
+        pybind11::arg("z"), pybind11::arg("rate"), pybind11::arg("tokens"));
+  m.def("softplus_gradients", &softplus_gradients,
+        "(grad_z, grad_rate, grad_tokens) of the softplus-gate scan", pybind11::arg("z"),
+        pybind11::arg("rate"), pybind11::arg("out"), pybind11::arg("grad_out"));
   m.def("fullscan_backward_softplus", &fullscan_backward_softplus,
         "fused backward of the softplus-gate scan: writes grad_z, grad_tokens and one "
         "d loss / d rate partial per row", pybind11::arg("z"), pybind11::arg("rate"),

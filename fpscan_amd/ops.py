@@ -173,8 +173,9 @@ class PScanChannelLast(torch.autograd.Function):
 
 
 def pscan_channel_last(gates: torch.Tensor, tokens: torch.Tensor) -> torch.Tensor:
-    """Differentiable scan of (batch, seqlen, dim) tensors along seqlen."""
-    return PScanChannelLast.apply(gates, tokens)
+    """Differentiable scan of (batch, seqlen, dim) tensors along seqlen: the computation of
+    ``PScanChannelLast.apply``, run by the extension's C++ autograd function (see ``pscan``)."""
+    return _load_extension().pscan_cl(gates, tokens)
 
 
 # ---------------------------------------------------------------------------------------
@@ -207,14 +208,8 @@ def scan_backward_softplus(
 ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """(grad_z, grad_rate, grad_tokens) of ``scan_forward_softplus`` (forward direction)
     given its output. grad_rate is float32 with rate's shape: the kernel writes one partial
-    sum per (batch, dim) row and the batch is summed here."""
-    ext = _load_extension()
-    grad_z = torch.empty_like(z)
-    grad_tokens = torch.empty_like(z)
-    B, D = z.shape[0], z.shape[1]
-    rows = torch.empty(B * D, dtype=torch.float32, device=z.device)
-    ext.fullscan_backward_softplus(z, rate, out, grad_out, grad_z, grad_tokens, rows)
-    return grad_z, rows.view(B, D).sum(0).view(rate.shape), grad_tokens
+    sum per (batch, dim) row and a second one sums the batch."""
+    return _load_extension().softplus_gradients(z, rate, out, grad_out)
 
 
 class PScanSoftplus(torch.autograd.Function):
@@ -236,8 +231,9 @@ class PScanSoftplus(torch.autograd.Function):
 
 def pscan_softplus(z: torch.Tensor, rate: torch.Tensor, tokens: torch.Tensor) -> torch.Tensor:
     """Differentiable ``pscan(torch.exp(-softplus(z) * rate[:, None]), tokens)`` with the
-    gates computed inside the kernels (forward and backward)."""
-    return PScanSoftplus.apply(z, rate, tokens)
+    gates computed inside the kernels (forward and backward): the computation of
+    ``PScanSoftplus.apply``, run by the extension's C++ autograd function (see ``pscan``)."""
+    return _load_extension().pscan_softplus(z, rate, tokens)
 
 
 # ---------------------------------------------------------------------------------------

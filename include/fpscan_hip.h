@@ -220,6 +220,11 @@ int fpscan_scan_bwd_softplus(const void* z, const float* rate, const void* out,
                              int64_t stride_b, int64_t stride_d,
                              int dtype, void* stream);
 
+/* grad_rate[d] = the sum over b of grad_rate_rows[b * dim + d] (fpscan_scan_bwd_softplus's
+ * partial sums; batch and dim at least 1), accumulated in double and rounded once. */
+int fpscan_sum_rate_rows(const float* grad_rate_rows, float* grad_rate, int64_t batch,
+                         int64_t dim, void* stream);
+
 /* Contraction scan, in place into `tokens` (the reference's Bx):
  * replaces dimwise_forward / dimwise_fwd / dimwise_pscan (csrc/main.cpp:10,
  * csrc/dimwise/dimwise.h:27-42, csrc/dimwise/dimwise_scan_final.cu:387-576).
