@@ -1139,10 +1139,17 @@ int run(const Args& a, void* workspace, size_t ws_bytes, hipStream_t stream) {
   // L8192 68.1 -> 64.8); fused-gate backward on rows of 16-32 sub-chunks at 16-256 MiB 11-25 %
   // (bf16 8192 rows of L8192 152.4 -> 117.4). Elsewhere 8 waves measured slower (2-9 % on
   // rows of 2-8 rounds at 128-256 MiB, up to 5 % below 16 MiB, where a call takes about 7 us)
-  // or even (the plain backward on rows of 16 at 128-256 MiB).
+  // or even (the plain backward on rows of 16 at 128-256 MiB). The plain backward takes 8
+  // waves on rows of any length at 16-128 MiB: two rows a CU hide each other's ring fill and
+  // drain at the row's ends, which shows once its gates and forward output come out of the
+  // memory-side cache (a training step: bf16 (1, 1024, 65536) 171.0 -> 164.3 us, (1, 512, 65536)
+  // 90.1 -> 85.0, fp32 (4, 1024, 8192) 166.4 -> 161.8; alone it is within 1.5 % either way, and
+  // at 192 MiB 1-4 % slower).
   const int64_t kib = a.rows * nsub;  // tensor size: a sub-chunk is 1 KiB
   const bool from16 = kib >= (16 << 10);
   const bool eight = (nsub >= 16 && nsub <= 64 && from16 && kib <= (64 << 10)) ||
+                     (kMode == kBwd && !Gp::kFused && nsub >= 16 && from16 &&
+                      kib <= (128 << 10)) ||
                      (kMode != kBwd && nsub == 16 && from16) ||
                      (Gp::kFused && kMode == kBwd && nsub >= 16 && nsub <= 32 && from16);
   if (eight) w = 8;
