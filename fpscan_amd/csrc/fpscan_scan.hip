@@ -1153,6 +1153,19 @@ int run(const Args& a, void* workspace, size_t ws_bytes, hipStream_t stream) {
                      (kMode != kBwd && nsub == 16 && from16) ||
                      (Gp::kFused && kMode == kBwd && nsub >= 16 && nsub <= 32 && from16);
   if (eight) w = 8;
+  // Rows of 8 sub-chunks in the forward and reverse from 16 to 256 MiB, and with the fused gates
+  // rows of 8 always and of 4 in the forward and reverse: half the waves, each with two
+  // sub-chunks in flight, so that a CU holds more rows at once and their loads, scans and stores
+  // overlap. Measured on MI355X (us, one round of w waves -> two of w / 2): bf16 (4, 1024, 4096)
+  // forward 18.7 -> 17.7, fp32 (8, 1024, 2048) 34.1 -> 32.6, 128 MiB 65.4 -> 64.3, 256 MiB 125.8 ->
+  // 125.3, but 512 MiB 260.4 -> 265.2 and at 4 MiB 5.5 -> 5.6; fused gates on rows of 8 forward /
+  // backward 19.4 / 31.6 -> 18.5 / 30.8 at 32 MiB, 67.0 / 112.7 -> 64.7 / 107.9 at 128 MiB, 130.8 /
+  // 224.6 -> 126.7 / 213.9 at 256 MiB, forward on rows of 4 19.8 -> 18.5 at 32 MiB and 133.8 ->
+  // 129.5 at 256 MiB (the backward there 1-2 % slower). The plain backward loses 2 % on rows of 8,
+  // and the plain forward is even on rows of 4 at 32 MiB and loses 3 % at 256 MiB.
+  if (Gp::kFused ? nsub == 8 || (nsub == 4 && kMode != kBwd)
+                 : kMode != kBwd && nsub == 8 && from16 && kib <= (256 << 10))
+    w = nsub / 2;
   int u_max = (w == 1 && kMode != kBwd) ? 4
               : (w == 16 && kMode != kBwd && nsub >= 8 * 16) ? 4
               : (w == 16 && (!Gp::kFused || kMode != kBwd) ? 3 : 2);

@@ -24,6 +24,34 @@ def test_long_rows_backward(dtype, rows, subs):
     _check(dtype, rows, subs)
 
 
+# half the waves: the plain forward on rows of 8 sub-chunks from 16 to 256 MiB
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("rows,subs", [(2047, 8), (2048, 8), (32768, 8), (32769, 8)], ids=str)
+def test_rows_of_eight_sub_chunks(dtype, rows, subs):
+    _check(dtype, rows, subs)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("reverse", [False, True], ids=["fwd", "rev"])
+@pytest.mark.parametrize("rows,subs", [(3, 4), (7, 8), (2048, 8)], ids=str)
+def test_softplus_rows_of_four_and_eight_sub_chunks(dtype, rows, subs, reverse):
+    L = subs * (1024 // torch.empty((), dtype=dtype).element_size())
+    gen = torch.Generator(device=DEVICE).manual_seed(rows)
+    z, x, go = (torch.randn((1, rows, L), generator=gen, device=DEVICE).to(dtype)
+                for _ in range(3))
+    rate = 0.1 * torch.rand(rows, generator=gen, device=DEVICE)
+    y = fpscan_amd.scan_forward_softplus(z, rate, x, reverse)
+    pick = torch.tensor(sorted({0, rows // 2, rows - 1}))
+    at = [t[:, pick].cpu() for t in (z, x, go)]
+    r = rate[pick].cpu()
+    check(y[:, pick].cpu(), oracle.scan_softplus_f64(at[0], r, at[1], reverse), dtype, "forward")
+    if not reverse:
+        gz, gr, gx = fpscan_amd.scan_backward_softplus(z, rate, y, go)
+        gz_ref, gr_ref, gx_ref = oracle.scan_bwd_softplus_f64(at[0], r, y[:, pick].cpu(), at[2])
+        check(gz[:, pick].cpu(), gz_ref, dtype, "grad_z")
+        check(gx[:, pick].cpu(), gx_ref, dtype, "grad_tokens")
+
+
 def _check(dtype, rows, subs):
     L = subs * (1024 // torch.empty((), dtype=dtype).element_size())
     gen = torch.Generator(device=DEVICE).manual_seed(rows)
