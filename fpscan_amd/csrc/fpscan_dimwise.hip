@@ -22,7 +22,8 @@
 //
 // Work decomposition: one workgroup per row; its waves are the sub-chunks (64 lanes x one
 // 16-byte vector per lane) of one chunk; a group is GL consecutive lanes, scanned with a
-// segmented DPP scan. v and r go through LDS; wave 0 selects (lane g for group g, W <= 32)
+// segmented DPP scan. v and r go through LDS; wave 0 selects (lane g for group g, W <= 32;
+// with 32 groups lanes g and g + 32 share its candidates)
 // and keeps the chunk carry in a register, so a chunk costs two barriers. The next chunk's
 // operands are in flight while a chunk is computed.
 #include <hip/hip_runtime.h>
@@ -86,6 +87,14 @@ __device__ __forceinline__ float load1(const void* p, int64_t i) {
   }
 }
 
+// Lanes 0..31: the value of lane + 32 (lanes 32..63 keep theirs).
+__device__ __forceinline__ float upper_half(float v) {
+  const unsigned int u = __builtin_bit_cast(unsigned int, v);
+  return __builtin_bit_cast(float, (unsigned int)__builtin_amdgcn_permlane32_swap(u, u, false, false)[1]);
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
 template <class E, int GL, int NW>
 __global__ void __launch_bounds__(64 * NW) dimwise_rows(const DwArgs a) {
   constexpr int V = E::V;
@@ -94,6 +103,8 @@ __global__ void __launch_bounds__(64 * NW) dimwise_rows(const DwArgs a) {
 
   __shared__ float v_lds[32];
   __shared__ float r_lds[32];
+  __shared__ __align__(16) float k_lds[32];
+  constexpr bool kHalves = NW * 64 / GL == 32;  // chunks of 32 groups
 
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -124,6 +135,7 @@ __global__ void __launch_bounds__(64 * NW) dimwise_rows(const DwArgs a) {
     if (w == 0) {
       wq = load1<E>(a.wq, d);
       if (lane < W) k = scale1p<E>(load1<E>(a.wk, d), load1<E>(a.bh, row * G + lane));
+      if (kHalves && lane < 32) k_lds[lane] = k;  // read by this wave only
     }
 
     u32x4 ring[2][2];
@@ -172,15 +184,45 @@ __global__ void __launch_bounds__(64 * NW) dimwise_rows(const DwArgs a) {
 
         if (w == 0) {
           // lane g selects for group g
-          const float vg = lane < W ? v_lds[lane] : 0.0f;
+          // With 32 groups the two halves of the wave take 16 candidates each, the later ones
+          // winning only if strictly larger, as in one pass over h. Every other wave of the
+          // row waits here, so the selection's length is the chunk's: measured on MI355X
+          // against one pass of 31 candidates with a readlane each, with the copy of Bx that
+          // precedes each timed call, fp32 (4, 512, 8192) 59.2 -> 55.6 us, bf16 (8, 256, 16384)
+          // 58.2 -> 54.8, (3, 100, 8192) 11.5 -> 10.1, (1, 64, 65536) 35.6 -> 24.4; full streams
+          // of long chunks are even (fp32 (10, 607, 16384) 344 -> 347).
+          const int g_sel = kHalves ? lane & 31 : lane;
+          const float vg = g_sel < W ? v_lds[g_sel] : 0.0f;
           const float q = scale1p<E>(wq, round_t<E>(vg));
           float best = kInit;
           int m = 0;
-          for (int h = 0; h < W - 1; ++h) {
-            const float s = round_t<E>(readlane(k, h) * q);
-            if (h < lane && s > best) {
-              best = s;
-              m = h;
+          if constexpr (kHalves) {
+            const int h0 = lane < 32 ? 0 : 16;
+#pragma unroll 1  // unrolled it takes more than 64 registers: one workgroup per CU, not two
+            for (int j = 0; j < 16; j += 4) {
+              const f32x4 kq = *reinterpret_cast<const f32x4*>(&k_lds[h0 + j]);
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const float s = round_t<E>(kq[i] * q);
+                if (h0 + j + i < g_sel && s > best) {
+                  best = s;
+                  m = h0 + j + i;
+                }
+              }
+            }
+            const float best_hi = upper_half(best);
+            const int m_hi = __builtin_bit_cast(int, upper_half(__builtin_bit_cast(float, m)));
+            if (best_hi > best) {
+              best = best_hi;
+              m = m_hi;
+            }
+          } else {
+            for (int h = 0; h < W - 1; ++h) {
+              const float s = round_t<E>(readlane(k, h) * q);
+              if (h < lane && s > best) {
+                best = s;
+                m = h;
+              }
             }
           }
           const float r = lane == 0 ? vg : fmaf(best, v_lds[m], vg);
