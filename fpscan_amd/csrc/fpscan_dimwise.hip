@@ -23,9 +23,9 @@
 // Work decomposition: one workgroup per row; its waves are the sub-chunks (64 lanes x one
 // 16-byte vector per lane) of one chunk; a group is GL consecutive lanes, scanned with a
 // segmented DPP scan. v and r go through LDS; wave 0 selects (lane g for group g, W <= 32;
-// with 32 groups lanes g and g + 32 share its candidates)
-// and keeps the chunk carry in a register, so a chunk costs two barriers. The next chunk's
-// operands are in flight while a chunk is computed.
+// with 32 groups lanes g and g + 32 share its candidates) and keeps the chunk carry in a
+// register, so a chunk costs two barriers. The next chunk's operands are in flight while a
+// chunk is computed.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

@@ -78,8 +78,11 @@ __device__ __forceinline__ int64_t row_offset(const Args& a, int64_t row) {
   return b * a.stride_b + d * a.stride_d;
 }
 
+template <bool kStream>
 __device__ __forceinline__ u32x4 ld16(const void* base, int64_t elem, int size) {
-  return *reinterpret_cast<const u32x4*>(static_cast<const char*>(base) + elem * size);
+  const u32x4* p = reinterpret_cast<const u32x4*>(static_cast<const char*>(base) + elem * size);
+  if constexpr (kStream) return __builtin_nontemporal_load(p);
+  return *p;
 }
 
 __device__ __forceinline__ void st16(void* base, int64_t elem, int size, u32x4 v) {
@@ -825,14 +828,32 @@ scan_tiles(const Args a, uint64_t* __restrict__ status, const int tpr_log2, cons
 }
 
 // ---------------------------------------------------------------------------------------
-// Short rows: G lanes per row (seqlen = G * V), 64/G rows per wave, 4 waves per block.
+// Short rows: G lanes per row (seqlen = G * V), 64/G rows per wave.
+//
+// kLarge, from kShortLargeBytes per tensor: one wave per block, so that every wave slot that
+// frees up takes its next rows at once, and nontemporal loads; below, 4 waves per block and
+// loads of the default policy, which find what the memory-side cache still holds of the
+// operands. Bound by HBM. Measured on MI355X, 4 waves and default loads -> 1 wave and
+// nontemporal ones, forward + backward (us): bf16 (64, 8192, 128), 128 MiB, 69.1 + 119.0 -> 62.4 +
+// 105.7, fp32 (64, 8192, 128), 256 MiB, 133.1 + 235.5 -> 121.6 + 211.5, (16, 8192, 128), 64 MiB,
+// 35.7 + 59.3 -> 32.0 + 54.2, softplus bf16 128 MiB 70.1 + 116.9 -> 63.9 + 107.0; but at 32 MiB bf16
+// (16, 4096, 256) 15.6 + 28.7 -> 17.0 + 28.0 (the calls' operands still cached), at 16 MiB 8.5 +
+// 13.3 -> 9.0 + 15.6. A training step with that cache full of other data to be written back: 128 MiB
+// 234 -> 174 (default loads push it out to HBM). Nontemporal loads with 4 waves: 64.6 + 111.4.
 // ---------------------------------------------------------------------------------------
-template <class E, int kMode, int G, class Gp = GatePlain>
-__global__ void __launch_bounds__(256) scan_short_rows(const Args a) {
+constexpr int64_t kShortLargeBytes = 64ll << 20;
+
+template <bool kLarge>
+constexpr int short_block_waves() {
+  return kLarge ? 1 : 4;
+}
+
+template <class E, int kMode, int G, class Gp, bool kLarge>
+__global__ void __launch_bounds__(64 * short_block_waves<kLarge>()) scan_short_rows(const Args a) {
   constexpr int V = E::V;
   constexpr bool kReverse = kMode != kFwd;
   constexpr int kRowsPerWave = 64 / G;
-  constexpr int kRowsPerBlock = 4 * kRowsPerWave;
+  constexpr int kRowsPerBlock = short_block_waves<kLarge>() * kRowsPerWave;
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -851,9 +872,9 @@ __global__ void __launch_bounds__(256) scan_short_rows(const Args a) {
     Slot<kMode> s;
     if (valid) {
       const int64_t e = base + (int64_t)vec * V;
-      s.v[0] = ld16(a.in0, e, E::kSize);
-      s.v[1] = ld16(a.in1, e, E::kSize);
-      if constexpr (kMode == kBwd) s.v[2] = ld16(a.in2, e, E::kSize);
+      s.v[0] = ld16<kLarge>(a.in0, e, E::kSize);
+      s.v[1] = ld16<kLarge>(a.in1, e, E::kSize);
+      if constexpr (kMode == kBwd) s.v[2] = ld16<kLarge>(a.in2, e, E::kSize);
     } else {
 #pragma unroll
       for (int i = 0; i < (kMode == kBwd ? 3 : 2); ++i) s.v[i] = u32x4{0u, 0u, 0u, 0u};
@@ -1058,13 +1079,13 @@ const void* long_kernel(int w, int u) {
   }
 }
 
-template <class E, int kMode, class Gp>
+template <class E, int kMode, class Gp, bool kLarge>
 const void* short_kernel(int g) {
   switch (g) {
-    case 4: return reinterpret_cast<const void*>(&scan_short_rows<E, kMode, 4, Gp>);
-    case 8: return reinterpret_cast<const void*>(&scan_short_rows<E, kMode, 8, Gp>);
-    case 16: return reinterpret_cast<const void*>(&scan_short_rows<E, kMode, 16, Gp>);
-    default: return reinterpret_cast<const void*>(&scan_short_rows<E, kMode, 32, Gp>);
+    case 4: return reinterpret_cast<const void*>(&scan_short_rows<E, kMode, 4, Gp, kLarge>);
+    case 8: return reinterpret_cast<const void*>(&scan_short_rows<E, kMode, 8, Gp, kLarge>);
+    case 16: return reinterpret_cast<const void*>(&scan_short_rows<E, kMode, 16, Gp, kLarge>);
+    default: return reinterpret_cast<const void*>(&scan_short_rows<E, kMode, 32, Gp, kLarge>);
   }
 }
 
@@ -1118,9 +1139,11 @@ int run(const Args& a, void* workspace, size_t ws_bytes, hipStream_t stream) {
   }
   if (L < kSub) {
     const int g = L / V;
-    const int64_t rows_per_block = 4 * (64 / g);
-    return launch(short_kernel<E, kMode, Gp>(g), (a.rows + rows_per_block - 1) / rows_per_block,
-                  256, a, stream);
+    const bool large = a.rows * L * E::kSize >= kShortLargeBytes;
+    const int waves = large ? short_block_waves<true>() : short_block_waves<false>();
+    const int64_t rows_per_block = waves * (64 / g);
+    return launch(large ? short_kernel<E, kMode, Gp, true>(g) : short_kernel<E, kMode, Gp, false>(g),
+                  (a.rows + rows_per_block - 1) / rows_per_block, 64 * waves, a, stream);
   }
   const int nsub = L / kSub;
   // Up to 16 waves share a row: each round then touches W KiB of each tensor contiguously

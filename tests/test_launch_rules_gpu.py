@@ -52,8 +52,18 @@ def test_softplus_rows_of_four_and_eight_sub_chunks(dtype, rows, subs, reverse):
         check(gx[:, pick].cpu(), gx_ref, dtype, "grad_tokens")
 
 
+# short rows (64 elements): one wave per block from 64 MiB per tensor, a last block that is
+# partly empty, and the size just below
+@pytest.mark.parametrize("dtype,rows", [(torch.float32, (1 << 18) - 1), (torch.float32, 1 << 18),
+                                        (torch.float32, (1 << 18) + 1),
+                                        (torch.bfloat16, (1 << 19) - 1),
+                                        (torch.bfloat16, (1 << 19) + 5)], ids=str)
+def test_short_rows_around_64_mib(dtype, rows):
+    _check(dtype, rows, 64 * torch.empty((), dtype=dtype).element_size() / 1024)
+
+
 def _check(dtype, rows, subs):
-    L = subs * (1024 // torch.empty((), dtype=dtype).element_size())
+    L = int(subs * (1024 // torch.empty((), dtype=dtype).element_size()))
     gen = torch.Generator(device=DEVICE).manual_seed(rows)
     g = torch.sigmoid(3 + torch.randn((1, rows, L), generator=gen, device=DEVICE)).to(dtype)
     x, go = (torch.randn((1, rows, L), generator=gen, device=DEVICE).to(dtype) for _ in range(2))
