@@ -85,8 +85,14 @@ __device__ __forceinline__ u32x4 ld16(const void* base, int64_t elem, int size) 
   return *p;
 }
 
+template <bool kStream>
 __device__ __forceinline__ void st16(void* base, int64_t elem, int size, u32x4 v) {
-  __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(static_cast<char*>(base) + elem * size));
+  u32x4* p = reinterpret_cast<u32x4*>(static_cast<char*>(base) + elem * size);
+  if constexpr (kStream) {
+    __builtin_nontemporal_store(v, p);
+  } else {
+    *p = v;
+  }
 }
 
 
@@ -848,7 +854,7 @@ constexpr int short_block_waves() {
   return kLarge ? 1 : 4;
 }
 
-template <class E, int kMode, int G, class Gp, bool kLarge>
+template <class E, int kMode, int G, class Gp, bool kLarge, int kKeep>
 __global__ void __launch_bounds__(64 * short_block_waves<kLarge>()) scan_short_rows(const Args a) {
   constexpr int V = E::V;
   constexpr bool kReverse = kMode != kFwd;
@@ -872,7 +878,7 @@ __global__ void __launch_bounds__(64 * short_block_waves<kLarge>()) scan_short_r
     Slot<kMode> s;
     if (valid) {
       const int64_t e = base + (int64_t)vec * V;
-      s.v[0] = ld16<kLarge>(a.in0, e, E::kSize);
+      s.v[0] = ld16<kLarge && kKeep != kKeepBoth>(a.in0, e, E::kSize);
       s.v[1] = ld16<kLarge>(a.in1, e, E::kSize);
       if constexpr (kMode == kBwd) s.v[2] = ld16<kLarge>(a.in2, e, E::kSize);
     } else {
@@ -893,8 +899,8 @@ __global__ void __launch_bounds__(64 * short_block_waves<kLarge>()) scan_short_r
     u32x4 o0, o1;
     finish_lane<E, kMode, Gp>(al, be, ysh, y_enter, o0, o1, &aux, &rate_sum);
     if (valid) {
-      st16(a.out0, base + (int64_t)vec * V, E::kSize, o0);
-      if constexpr (kMode == kBwd) st16(a.out1, base + (int64_t)vec * V, E::kSize, o1);
+      st16<!kLarge || kKeep == kKeepNone>(a.out0, base + (int64_t)vec * V, E::kSize, o0);
+      if constexpr (kMode == kBwd) st16<true>(a.out1, base + (int64_t)vec * V, E::kSize, o1);
     }
     if constexpr (Gp::kFused && kMode == kBwd) {
       const float tot = segment_sum<G>(rate_sum, sl);  // the row's last lane holds its sum
@@ -1079,13 +1085,13 @@ const void* long_kernel(int w, int u) {
   }
 }
 
-template <class E, int kMode, class Gp, bool kLarge>
+template <class E, int kMode, class Gp, bool kLarge, int kKeep>
 const void* short_kernel(int g) {
   switch (g) {
-    case 4: return reinterpret_cast<const void*>(&scan_short_rows<E, kMode, 4, Gp, kLarge>);
-    case 8: return reinterpret_cast<const void*>(&scan_short_rows<E, kMode, 8, Gp, kLarge>);
-    case 16: return reinterpret_cast<const void*>(&scan_short_rows<E, kMode, 16, Gp, kLarge>);
-    default: return reinterpret_cast<const void*>(&scan_short_rows<E, kMode, 32, Gp, kLarge>);
+    case 4: return reinterpret_cast<const void*>(&scan_short_rows<E, kMode, 4, Gp, kLarge, kKeep>);
+    case 8: return reinterpret_cast<const void*>(&scan_short_rows<E, kMode, 8, Gp, kLarge, kKeep>);
+    case 16: return reinterpret_cast<const void*>(&scan_short_rows<E, kMode, 16, Gp, kLarge, kKeep>);
+    default: return reinterpret_cast<const void*>(&scan_short_rows<E, kMode, 32, Gp, kLarge, kKeep>);
   }
 }
 
@@ -1142,7 +1148,8 @@ int run(const Args& a, void* workspace, size_t ws_bytes, hipStream_t stream) {
     const bool large = a.rows * L * E::kSize >= kShortLargeBytes;
     const int waves = large ? short_block_waves<true>() : short_block_waves<false>();
     const int64_t rows_per_block = waves * (64 / g);
-    return launch(large ? short_kernel<E, kMode, Gp, true>(g) : short_kernel<E, kMode, Gp, false>(g),
+    return launch(large ? short_kernel<E, kMode, Gp, true, kKeep>(g)
+                        : short_kernel<E, kMode, Gp, false, kKeepNone>(g),
                   (a.rows + rows_per_block - 1) / rows_per_block, 64 * waves, a, stream);
   }
   const int nsub = L / kSub;
@@ -1240,8 +1247,9 @@ int dispatch(int dtype, const Args& a, void* ws, size_t ws_bytes, hipStream_t st
 // so those stream. With the softplus gates only the output is kept (128 MiB 183.3 -> 180.2, 64
 // MiB fp32 93.1 -> 91.7): keeping z as well measured 8 % slower with the cache full. A forward
 // alone gains nothing (138.5 us streamed, 144.5 with both at 256 MiB), so fpscan_scan_fwd
-// streams, and so do rows shorter than a sub-chunk (keeping measured 2 % slower at 128 MiB,
-// bf16 (64, 8192, 128)).
+// streams. Rows shorter than a sub-chunk keep from kShortLargeBytes (bf16 (64, 8192, 128) 169.2 ->
+// 156.0, fp32 (16, 8192, 128) 85.6 -> 80.0, softplus bf16 171.7 -> 166.5); below, their loads have
+// the default policy anyway and the output streams (keeping it measured 2 % slower).
 constexpr int64_t kKeepMaxBytes = 128ll << 20;
 
 template <class Gp>

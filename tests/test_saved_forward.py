@@ -17,11 +17,10 @@ gpu = [pytest.mark.gpu,
        pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device (MI355X)")]
 
 # (rows, sub-chunks per row): waves per row 1 (four rows a block, one row a block), 2, 4, 8 and
-# 16, the ring depths, short rows (0: a row of half a sub-chunk), and tensors of 128 MiB and
-# more, on both sides of the line between keeping the output and the gates and the gates alone
-# (a sub-chunk is 1 KiB)
-ROWS = [(6, 0), (6, 1), (32768, 1), (5, 2), (5, 4), (5, 8), (5, 16), (2048, 16), (3, 32),
-        (3, 128), (1024, 128), (1025, 128)]
+# 16, the ring depths, short rows (0: a row of half a sub-chunk; around 64 MiB), and tensors on
+# both sides of 128 MiB, where keeping ends (a sub-chunk is 1 KiB)
+ROWS = [(6, 0), (131071, 0), (131072, 0), (6, 1), (32768, 1), (5, 2), (5, 4), (5, 8), (5, 16),
+        (2048, 16), (3, 32), (3, 128), (1024, 128), (1025, 128)]
 
 
 @pytest.mark.parametrize("softplus", [False, True], ids=["gates", "softplus"])
