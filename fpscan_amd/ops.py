@@ -14,6 +14,9 @@ Drop-in for ``fpscan/ops.py`` of saeeddhqan/fpscan:
 * ``pscan`` mirrors fpscan/ops.py:86-87; the autograd function it applies is the C++ twin of
   ``PScan`` in the extension (same saved tensors, same kernels), which spares the engine a
   Python call in the forward and in the backward. ``PScan.apply`` keeps working.
+  ``pscan_channel_last`` and ``pscan_softplus`` have C++ twins likewise.
+* The autograd forwards call the extension's ``*_saved`` forms: the same results, with the
+  gates and the output left in the memory-side cache for the backward while they fit.
 """
 from __future__ import annotations
 
