@@ -1396,6 +1396,7 @@ ClBlockPlan plan_cl_blocks(int64_t batch, int64_t seqlen, int64_t dim, int64_t s
   t.chains = batch * t.npan;
   t.r = bwd && !t.shared && t.chains >= kClbFewChains ? 4 : 8;
   const int64_t steps = (int64_t)t.groups * t.r;
+  if (seqlen > INT32_MAX - steps) return t;  // the last tile's end stays within 32 bits
   t.nseg = (seqlen + steps - 1) / steps;
   t.ntiles = t.chains * t.nseg;
   const int64_t words = t.ntiles * t.cv * vec * 3 / 2 + kStatusExtraWords;
