@@ -857,6 +857,20 @@ scan_cl_tiles(const ClArgs a, uint64_t* __restrict__ status, const int64_t ntile
 // then all chains' tile 1, ...), so a tile waits only for tiles that running workgroups hold.
 // With a single tile per chain there is nothing to wait for, and no workspace.
 //
+// Values that leave fp32's range: a tile's map is a product over up to 2048 gates, so gates
+// above 1 can overflow it (1.42 over 256 steps) where the states themselves are finite, and
+// Inf x 0 would then make the rest of the chain NaN; a product that underflows does the same to
+// a state of Inf. A map applied to a non-finite value never gives a finite one, so the results
+// tell: a carry whose composition is not finite is replaced by the predecessor's end value, and
+// a column whose state leaves the range inside the tile has the values entering its groups
+// computed again, one step after the other. So every value is what the serial recurrence gives
+// wherever the products over one lane's R steps are finite. Every tile publishes its end value
+// (a composed one that is not finite only once it is settled); a NaN in it is passed on at
+// once, as it makes every later state of its chain NaN in the recurrence too. Only chains with
+// such values pay, by waiting for one tile after the other: bf16 (1, 65536, 1024) 86 -> 384 us
+// with gates of 1.5, 417 with an Inf early on. The tests themselves cost up to 1 % from 30 MiB,
+// 0.1-0.2 us of calls of 5-15 us.
+//
 // Against scan_cl_tiles (one 1024-thread workgroup per CU with a ring of tiles): no start-up
 // chain of claims, no ring to fill and drain, so a call of tens of microseconds is shorter;
 // the other workgroups of the CU cover a tile's waits instead of the ring. The bound is the
@@ -885,6 +899,10 @@ constexpr int kClbStream = 0;
 constexpr int kClbSaved = 1;
 constexpr int kClbShared = 2;
 
+__device__ __forceinline__ bool is_finite(float v) {
+  return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u;
+}
+
 template <class E, int kMode, int R, int kPol>
 __global__ void __launch_bounds__(kClbThreads, (kMode == kBwd && R == 8) ? 3 : 4)
 scan_cl_blocks(const ClArgs a, uint64_t* __restrict__ status, const int64_t ntiles) {
@@ -899,6 +917,7 @@ scan_cl_blocks(const ClArgs a, uint64_t* __restrict__ status, const int64_t ntil
   __shared__ f32x4 maps[V / 2][kClbThreads];    // plane i: columns 2i, 2i+1 of the vector
   __shared__ f32x4 entry[V / 4][kClbThreads];   // plane j: columns 4j..4j+3
   __shared__ int64_t claimed;
+  __shared__ int serial;  // set if any column has to be computed serially
 
   const int tid = threadIdx.x;
   const int cv = a.cv;
@@ -1009,17 +1028,21 @@ scan_cl_blocks(const ClArgs a, uint64_t* __restrict__ status, const int64_t ntil
 #pragma unroll
     for (int i = 0; i < V / 2; ++i)
       maps[i][tid] = f32x4{A[2 * i], B[2 * i], A[2 * i + 1], B[2 * i + 1]};
+    if (tid == 0) serial = 0;
   }
   lds_barrier();
 
   // (2) one thread per column: aggregate, look-back, the value entering each group
+  const uint32_t ends_off = (uint32_t)(nagg * sizeof(uint64_t));
+  bool end_due = false;  // the end value is published after the enter loop, or the serial pass
   if (tid < ncols) {
     const int h = tid & 1;
     const int qi = (tid >> 1) / cv;
     const int qc = (tid >> 1) - qi * cv;
-    const f32x2* col_maps = reinterpret_cast<const f32x2*>(&maps[qi][qc]) + h;  // stride 2 cv
+    f32x2* col_maps = reinterpret_cast<f32x2*>(&maps[qi][qc]) + h;  // stride 2 cv
     float carry = 0.0f;
     if (chained) {
+      bool keep = false;  // the carry stands even if it is not finite
       float A = 1.0f, B = 0.0f;
 #pragma unroll 4
       for (int i = 0; i < a.groups; ++i) {
@@ -1029,7 +1052,6 @@ scan_cl_blocks(const ClArgs a, uint64_t* __restrict__ status, const int64_t ntil
       }
       const Rsrc st = __builtin_amdgcn_make_buffer_rsrc(
           status, (short)0, (int)((nstatus + kStatusExtraWords) * sizeof(uint64_t)), kRsrcWord3);
-      const uint32_t ends_off = (uint32_t)(nagg * sizeof(uint64_t));
       if (tile != a.skip_publish && seg + 1 < a.nseg)
         status_store(st, (uint32_t)((tile * ncols + tid) * sizeof(uint64_t)), pack_map(A, B));
       if (seg > 0) {
@@ -1046,6 +1068,7 @@ scan_cl_blocks(const ClArgs a, uint64_t* __restrict__ status, const int64_t ntil
             ends_off + (uint32_t)(((tile - (int64_t)(K + 1) * nch) * ncols + tid) *
                                   sizeof(uint32_t));
         end = end_load(st, seg > K ? end_at : kNoOffset);
+        bool gave_up = false;
         if (__builtin_amdgcn_ballot_w64(agg_missing(words, na) ||
                                         (seg > K && end == kEndNotPublished)) != 0) {
           const bool overran = __hip_atomic_load(status + nstatus, __ATOMIC_RELAXED,
@@ -1071,6 +1094,7 @@ scan_cl_blocks(const ClArgs a, uint64_t* __restrict__ status, const int64_t ntil
                 __hip_atomic_fetch_add(&g_cl_overruns, 1ull, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT);
               }
+              gave_up = true;
               break;
             }
           }
@@ -1080,27 +1104,109 @@ scan_cl_blocks(const ClArgs a, uint64_t* __restrict__ status, const int64_t ntil
             words[j] = words[j] == kNotPublished ? kPoisonMap : words[j];
           end = end == kEndNotPublished ? kPoisonValue : end;
         }
-        carry = seg > K ? __uint_as_float(end) : 0.0f;
+        const float past = seg > K ? __uint_as_float(end) : 0.0f;
+        carry = past;
 #pragma unroll
         for (int j = K - 1; j >= 0; --j)
           if (j < na)
             carry = fmaf(__uint_as_float((uint32_t)words[j]), carry,
                          __uint_as_float((uint32_t)(words[j] >> 32)));
+        keep = past != past || gave_up;
       }
-      if (seg + K + 1 < a.nseg)
-        end_store(st, ends_off + (uint32_t)((tile * ncols + tid) * sizeof(uint32_t)),
-                  canonical_bits(fmaf(A, carry, B)));
+      // published at once where it is finite; the test stands where NaNs were canonicalised
+      const uint32_t end_off =
+          seg + 1 < a.nseg ? ends_off + (uint32_t)((tile * ncols + tid) * sizeof(uint32_t))
+                           : kNoOffset;
+      const float e = fmaf(A, carry, B);
+      end_store(st, is_finite(e) ? end_off : kNoOffset, __float_as_uint(e));
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(!is_finite(e)) != 0, 0)) {
+        const bool again = seg > 0 && !is_finite(carry) && !keep;
+        const uint32_t* prev = reinterpret_cast<const uint32_t*>(status) + ends_off / 4 +
+                               (tile - nch) * ncols;
+        uint32_t v = kEndNotPublished;
+        for (int it = 0;; ++it) {
+          if (again && v == kEndNotPublished)
+            v = __hip_atomic_load(prev + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (__builtin_amdgcn_ballot_w64(again && v == kEndNotPublished) == 0) break;
+          if (it >= 8 * (int64_t)a.spin_limit) {  // here the chain's tiles follow one another
+            if ((tid & 63) == 0) {
+              __hip_atomic_fetch_add(status + nstatus, 1ull, __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_AGENT);
+              __hip_atomic_fetch_add(&g_cl_overruns, 1ull, __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_AGENT);
+            }
+            break;
+          }
+          __builtin_amdgcn_s_sleep(1);
+        }
+        if (again) carry = __uint_as_float(v == kEndNotPublished ? kPoisonValue : v);
+        if (!is_finite(e) && seg + 1 < a.nseg) {
+          const float e2 = fmaf(A, carry, B);
+          end_due = !is_finite(e2) && carry == carry;
+          if (!end_due) end_store(st, end_off, canonical_bits(e2));
+        }
+      }
     }
     const int e = 2 * qi + h;
     float* enter = reinterpret_cast<float*>(&entry[e / 4][qc]) + e % 4;  // stride 4 cv
+    const float entering = carry;
 #pragma unroll 4
     for (int i = 0; i < a.groups; ++i) {
       enter[4 * i * cv] = carry;
       const f32x2 m = col_maps[2 * i * cv];
       carry = fmaf(m.x, carry, m.y);
     }
+    // wrong only where the maps left the range: a NaN stays one, an Inf that is left at the end
+    // was one throughout
+    if (!is_finite(carry) && (is_finite(entering) || (entering == entering && carry != carry))) {
+      col_maps[0].y = carry;  // marks the column; the serial pass leaves its end value here
+      serial = 1;
+    } else if (end_due) {
+      __hip_atomic_store(reinterpret_cast<uint32_t*>(status) + ends_off / 4 + tile * ncols + tid,
+                         canonical_bits(carry), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      end_due = false;
+    }
   }
   lds_barrier();
+
+  // the marked columns serially: one group of steps after the other
+  if (__builtin_expect(__builtin_amdgcn_readfirstlane(serial) != 0, 0)) {
+    for (int i = 0; i < a.groups; ++i) {
+      if (g == i) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) asm volatile("" : "+v"(v0[r]), "+v"(v1[r]));
+        float y[V];
+#pragma unroll
+        for (int e = 0; e < V; ++e) y[e] = entry[e / 4][tid][e % 4];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          float ga[V], xb[V];
+          E::unpack(v0[r], ga);
+          E::unpack(v1[r], xb);
+#pragma unroll
+          for (int e = 0; e < V; ++e)
+            y[e] = fmaf(r == 0 && first ? 1.0f : ga[e], y[e], xb[e]);
+        }
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+          float* mark = reinterpret_cast<float*>(&maps[e / 2][c]) + 2 * (e % 2) + 1;
+          if (!is_finite(*mark)) {
+            if (i + 1 < a.groups)
+              reinterpret_cast<float*>(&entry[e / 4][tid + cv])[e % 4] = y[e];
+            else
+              *mark = y[e];
+          }
+        }
+      }
+      lds_barrier();
+    }
+    if (end_due) {
+      const int qi = (tid >> 1) / cv;
+      const f32x2* at = reinterpret_cast<const f32x2*>(&maps[qi][(tid >> 1) - qi * cv]) + (tid & 1);
+      __hip_atomic_store(reinterpret_cast<uint32_t*>(status) + ends_off / 4 + tile * ncols + tid,
+                         canonical_bits(at->y), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
 
   // (3) re-run the steps from the value entering the lane's group; the operands are unpacked
   // again (left to the compiler, their fp32 forms would be held across both barriers)
