@@ -470,8 +470,11 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> softplus_gradients(const at::Tens
   if (B == 0 || D == 0) return {grad_z, at::zeros_like(rate), grad_tokens};
   at::Tensor grad_rate = at::empty_like(rate);
   c10::hip::HIPGuardMasqueradingAsCUDA guard(z.device());
-  check_status(fpscan_sum_rate_rows(rows.data_ptr<float>(), grad_rate.data_ptr<float>(), B, D,
-                                    launch_stream(z)));
+  const size_t ws_bytes = fpscan_sum_rate_workspace_bytes(B, D);
+  at::Tensor ws = workspace(ws_bytes, z);
+  check_status(fpscan_sum_rate_rows_ws(rows.data_ptr<float>(), grad_rate.data_ptr<float>(), B, D,
+                                       ws_bytes ? ws.data_ptr() : nullptr, ws_bytes,
+                                       launch_stream(z)));
   return {grad_z, grad_rate, grad_tokens};
 }
 

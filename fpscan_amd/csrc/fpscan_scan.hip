@@ -909,30 +909,77 @@ __global__ void __launch_bounds__(64 * short_block_waves<kLarge>()) scan_short_r
   }
 }
 
-// Sum over the batch of the fused backward's per-row partial sums of d loss / d rate: a block
-// takes 64 channels, four waves a quarter of the batch each (the rows of one batch are
-// consecutive, so a wave reads 256 contiguous bytes a step). Bound by the launch and a few
-// load latencies: 3.8 us for 64 rows of 256 channels and 4.0 for 4 of 1024, as torch.sum takes on
-// the device (3.9), which adds its own host time to every step.
-constexpr int kSumWaves = 4;
-__global__ void __launch_bounds__(64 * kSumWaves)
-sum_rate_rows(const float* __restrict__ rows, float* __restrict__ out, int64_t batch,
-              int64_t dim) {
-  __shared__ double part[kSumWaves][64];
-  const int lane = threadIdx.x & 63;
-  const int w = threadIdx.x >> 6;
-  const int64_t d = (int64_t)blockIdx.x * 64 + lane;
+// Sum over the batch of the fused backward's per-row partial sums of d loss / d rate, in double
+// and in a fixed order. A block of 256 threads takes C channels (64, or the power of two that
+// holds fewer) of a slice of the batch; consecutive threads take consecutive channels, then
+// batches, so a wave reads whole lines. Long batches take two launches: the sums of up to
+// kSumMaxSlices slices, then their sum (In = double). Bound by the launch and a few load
+// latencies up to kSumSingle batches a thread, then by latencies per slice. Measured on MI355X
+// with one launch for every batch -> this (us; torch.sum in brackets): (64, 256) 3.0 -> 3.1,
+// (512, 128) 3.9 -> 4.2, (1024, 256) 6.5 -> 5.2 (9.5), (4096, 64) 21.9 -> 5.2 (8.8), (65536, 64)
+// 679 -> 9.1 (14.2), (262144, 1) 1583 -> 5.7 (9.8).
+constexpr int kSumThreads = 256;
+constexpr int kSumSingle = 128;     // batches per thread that one launch takes
+constexpr int kSumSlice = 32;       // batches per thread of a slice, at least
+constexpr int kSumMaxSlices = 256;
+constexpr int64_t kSumMaxDim = ((int64_t)1 << 31) - 64;
+
+template <class In, class Out>
+__global__ void __launch_bounds__(kSumThreads)
+sum_rate_rows(const In* __restrict__ rows, Out* __restrict__ out, const int64_t batch,
+              const int64_t dim, const int log2_c, const int64_t slice) {
+  __shared__ double part[kSumThreads];
+  const int tid = threadIdx.x;
+  const int slots = kSumThreads >> log2_c;
+  const int64_t d = ((int64_t)blockIdx.x << log2_c) + (tid & ((1 << log2_c) - 1));
+  const int64_t b0 = (int64_t)blockIdx.y * slice;
+  const int64_t b1 = b0 + slice < batch ? b0 + slice : batch;
   double sum = 0.0;
   if (d < dim) {
 #pragma unroll 8
-    for (int64_t b = w; b < batch; b += kSumWaves) sum += (double)rows[b * dim + d];
+    for (int64_t b = b0 + (tid >> log2_c); b < b1; b += slots) sum += (double)rows[b * dim + d];
   }
-  part[w][lane] = sum;
+  part[tid] = sum;
   __syncthreads();
-  if (w == 0 && d < dim) {
-    for (int i = 1; i < kSumWaves; ++i) sum += part[i][lane];
-    out[d] = (float)sum;
+  for (int half = slots / 2; half >= 4; half /= 2) {
+    if ((tid >> log2_c) < half) part[tid] += part[tid + (half << log2_c)];
+    __syncthreads();
   }
+  if (tid < 1 << log2_c && d < dim) {  // four sums are left
+    for (int i = 1; i < 4; ++i) sum = (i == 1 ? part[tid] : sum) + part[tid + (i << log2_c)];
+    out[blockIdx.y * dim + d] = (Out)sum;
+  }
+}
+
+struct SumPlan {
+  int log2_c;
+  int64_t slice, slices;
+  size_t bytes;  // workspace: a double per slice and channel; 0 with one launch
+};
+
+SumPlan plan_sum(int64_t batch, int64_t dim) {
+  SumPlan p{0, batch, 1, 0};
+  while (p.log2_c < 6 && ((int64_t)1 << p.log2_c) < dim) ++p.log2_c;
+  const int64_t slots = kSumThreads >> p.log2_c;
+  if (batch <= slots * kSumSingle) return p;
+  p.slice = slots * kSumSlice;
+  if ((batch + p.slice - 1) / p.slice > kSumMaxSlices)
+    p.slice = (batch + kSumMaxSlices - 1) / kSumMaxSlices;
+  p.slices = (batch + p.slice - 1) / p.slice;
+  p.bytes = (size_t)p.slices * (size_t)dim * sizeof(double);
+  return p;
+}
+
+template <class In, class Out>
+int launch_sum(const In* rows, Out* out, int64_t batch, int64_t dim, int log2_c, int64_t slice,
+               int64_t slices, hipStream_t stream) {
+  void* args[] = {&rows, &out, &batch, &dim, &log2_c, &slice};
+  const unsigned blocks = (unsigned)((dim + ((int64_t)1 << log2_c) - 1) >> log2_c);
+  return hipLaunchKernel(reinterpret_cast<const void*>(&sum_rate_rows<In, Out>),
+                         dim3(blocks, (unsigned)slices), dim3(kSumThreads), args, 0,
+                         stream) == hipSuccess
+             ? FPSCAN_OK
+             : FPSCAN_ERR_LAUNCH;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1499,14 +1546,26 @@ int fpscan_scan_bwd_softplus(const void* z, const float* rate, const void* out,
 
 int fpscan_sum_rate_rows(const float* grad_rate_rows, float* grad_rate, int64_t batch,
                          int64_t dim, void* stream) {
-  if (batch < 1 || dim < 1 || dim > ((int64_t)1 << 31) - 64) return FPSCAN_ERR_SHAPE;
+  return fpscan_sum_rate_rows_ws(grad_rate_rows, grad_rate, batch, dim, nullptr, 0, stream);
+}
+
+size_t fpscan_sum_rate_workspace_bytes(int64_t batch, int64_t dim) {
+  return batch < 1 || dim < 1 || dim > kSumMaxDim ? 0 : plan_sum(batch, dim).bytes;
+}
+
+int fpscan_sum_rate_rows_ws(const float* grad_rate_rows, float* grad_rate, int64_t batch,
+                            int64_t dim, void* workspace, size_t workspace_bytes, void* stream) {
+  if (batch < 1 || dim < 1 || dim > kSumMaxDim) return FPSCAN_ERR_SHAPE;
   if (!grad_rate_rows || !grad_rate) return FPSCAN_ERR_NULL;
-  void* args[] = {&grad_rate_rows, &grad_rate, &batch, &dim};
-  return hipLaunchKernel(reinterpret_cast<const void*>(&sum_rate_rows),
-                         dim3((unsigned)((dim + 63) / 64)), dim3(64 * kSumWaves), args, 0,
-                         static_cast<hipStream_t>(stream)) == hipSuccess
-             ? FPSCAN_OK
-             : FPSCAN_ERR_LAUNCH;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const SumPlan p = plan_sum(batch, dim);
+  if (p.bytes == 0 || workspace == nullptr || workspace_bytes < p.bytes)
+    return launch_sum(grad_rate_rows, grad_rate, batch, dim, p.log2_c, batch, 1, s);
+  double* part = static_cast<double*>(workspace);
+  const int st = launch_sum(grad_rate_rows, part, batch, dim, p.log2_c, p.slice, p.slices, s);
+  return st != FPSCAN_OK ? st
+                         : launch_sum(static_cast<const double*>(part), grad_rate, p.slices, dim,
+                                      p.log2_c, p.slices, 1, s);
 }
 
 size_t fpscan_workspace_bytes(int64_t batch, int64_t dim, int64_t seqlen, int dtype, int op) {

@@ -225,6 +225,14 @@ int fpscan_scan_bwd_softplus(const void* z, const float* rate, const void* out,
 int fpscan_sum_rate_rows(const float* grad_rate_rows, float* grad_rate, int64_t batch,
                          int64_t dim, void* stream);
 
+/* fpscan_sum_rate_rows with a workspace of fpscan_sum_rate_workspace_bytes() bytes (8-byte aligned,
+ * not used by any call in flight): batches of more than some hundred rows per channel are then
+ * summed in slices by many workgroups. With none (or a smaller one) one launch takes the whole
+ * batch: the same sum up to the last bit of its double, slower. 0 bytes: nothing is needed. */
+size_t fpscan_sum_rate_workspace_bytes(int64_t batch, int64_t dim);
+int fpscan_sum_rate_rows_ws(const float* grad_rate_rows, float* grad_rate, int64_t batch,
+                            int64_t dim, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Contraction scan, in place into `tokens` (the reference's Bx):
  * replaces dimwise_forward / dimwise_fwd / dimwise_pscan (csrc/main.cpp:10,
  * csrc/dimwise/dimwise.h:27-42, csrc/dimwise/dimwise_scan_final.cu:387-576).

@@ -62,6 +62,45 @@ def test_rate_gradient_is_the_batch_sum(batch, dim):
     assert ((grad_rate.double() - want).abs() <= 2.0 ** -24 * want.abs() + 1e-14).all()
 
 
+# one launch, two with a last slice that is short, and the most slices; channels that fill no wave
+@pytest.mark.parametrize("batch,dim", [(512, 64), (513, 64), (513, 65), (40000, 40), (32769, 1),
+                                       (100003, 3)], ids=str)
+def test_rate_gradient_of_long_batches(batch, dim):
+    gen = torch.Generator(device=DEVICE).manual_seed(batch)
+    rate = 0.1 * torch.rand(dim, generator=gen, device=DEVICE)
+    z, x, go = (torch.randn((batch, dim, 32), generator=gen, device=DEVICE) for _ in range(3))
+    rows = torch.empty(batch * dim, device=DEVICE)
+    ops._load_extension().fullscan_backward_softplus(z, rate, x, go, torch.empty_like(z),
+                                                     torch.empty_like(z), rows)
+    _, grad_rate, _ = fpscan_amd.scan_backward_softplus(z, rate, x, go)
+    rows = rows.view(batch, dim).double()
+    # one rounding to fp32, and the double sums' own order
+    bound = 2.0 ** -24 * rows.sum(0).abs() + batch * 2.0 ** -52 * rows.abs().sum(0)
+    assert ((grad_rate.double() - rows.sum(0)).abs() <= bound).all()
+
+
+def test_rate_gradient_of_a_long_batch_costs_less_than_the_scan():
+    z, out, go = (torch.randn((65536, 64, 32), device=DEVICE).bfloat16() for _ in range(3))
+    rate = 0.1 * torch.rand(64, device=DEVICE)
+    gz, gx, rows = torch.empty_like(z), torch.empty_like(z), torch.empty(65536 * 64, device=DEVICE)
+
+    def seconds(call):
+        times = []
+        for _ in range(4):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(5):
+                call()
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    scan = seconds(lambda: ops._load_extension().fullscan_backward_softplus(z, rate, out, go, gz,
+                                                                            gx, rows))
+    assert seconds(lambda: fpscan_amd.scan_backward_softplus(z, rate, out, go)) < 2 * scan
+
+
 def test_empty_batch_has_zero_rate_gradient():
     z = torch.empty(0, 5, 64, device=DEVICE)
     gz, gr, gx = fpscan_amd.scan_backward_softplus(z, torch.rand(5, device=DEVICE), z, z)
