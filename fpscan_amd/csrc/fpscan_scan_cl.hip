@@ -1509,6 +1509,20 @@ ClBlockPlan plan_cl_blocks(int64_t batch, int64_t seqlen, int64_t dim, int64_t s
   if (t.ntiles > INT32_MAX / kClbThreads || words * (int64_t)sizeof(uint64_t) > INT32_MAX ||
       (steps + 2) * stride_t * size > INT32_MAX)
     return t;
+  // A sequence within one tile leaves groups of the workgroup idle, which cost as much as busy
+  // ones, while the one pass costs a load latency per ring of steps. Measured on MI355X with the
+  // one pass -> this kernel at every length (us): forward, 256 chains of 16 / 32 / 64 steps (bf16)
+  // 5.0 / 5.7 / 9.3 -> 4.9 / 5.2 / 5.4, 1024 chains 5.1 / 6.1 / 10.7 -> 7.8 / 7.9 / 8.3, 3968
+  // chains of 32 / 64 / 96 10.7 / 27.2 / 29.2 -> 22.3 / 24.9 / 29.7; backward with R = 4, 512
+  // chains of 8 / 16 / 32 5.1 / 5.4 / 8.7 -> 5.2 / 5.6 / 5.9, 2048 chains of 16 / 32 / 64 6.5 / 10.2 /
+  // 19.4 -> 11.0 / 12.0 / 19.4; off the lines (R = 8), 1020 chains of 32 / 64 10.1 / 16.4 -> 13.3 /
+  // 17.4. At 5 steps, bf16 (62, 5, 3248) 3.9 + 4.3 -> 16.3 + 23.3.
+  if (t.nseg == 1) {
+    int64_t least = t.chains / (t.r == 4 ? 32 : 20);
+    if (least < (bwd ? 16 : 32)) least = bwd ? 16 : 32;
+    if (least > 96) least = 96;
+    if (seqlen < least) return t;
+  }
   const bool enough_strips = batch * ((nv + 63) / 64) >= kClMinTasks;
   if (t.shared ? enough_strips && t.nseg < 2
                : enough_strips || batch * seqlen * dim * size >= kClbMaxBytes)

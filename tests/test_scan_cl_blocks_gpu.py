@@ -64,6 +64,53 @@ def test_exact_on_integer_data(dtype, shape):
     assert bits_equal(gg.cpu(), torch.from_numpy(gg_ref).to(dtype))
 
 
+# around the length from which a sequence within one tile takes a block: 32 steps (the backward 16),
+# more with many chains, 96 at most; chains of 8 vectors on the lines, of up to 8 off them
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("shape", [(1, 15, 8), (1, 16, 8), (1, 31, 8), (1, 32, 8), (2, 31, 33),
+                                   (2, 32, 33), (16, 51, 8 * 64), (16, 52, 8 * 64),
+                                   (30, 95, 8 * 64), (30, 96, 8 * 64)], ids=str)
+def test_short_sequences(dtype, shape):
+    shape = _shape(shape, dtype)
+    g, x = cl_inputs(*shape, dtype, seed=3)
+    go = torch.randn(shape, generator=torch.Generator().manual_seed(5)).to(dtype)
+    y = fpscan_amd.scan_forward_channel_last(g.to(DEVICE), x.to(DEVICE))
+    check(y, oracle.scan_f64_channel_last(g, x), dtype, "forward")
+    gg, gx = fpscan_amd.scan_backward_channel_last(g.to(DEVICE), y, go.to(DEVICE))
+    gg_ref, gx_ref = oracle.scan_bwd_f64_channel_last(g, y.cpu(), go)
+    check(gx, gx_ref, dtype, "grad_tokens")
+    check(gg, gg_ref, dtype, "grad_gates")
+
+
+@pytest.mark.parametrize("shape", [(62, 5, 3248), (24, 1, 5856), (134, 8, 1280)], ids=str)
+def test_a_few_steps_cost_no_more_than_the_one_pass(shape):
+    g, x, go = (torch.rand(shape, device=DEVICE).bfloat16() for _ in range(3))
+    out, gg, gx = (torch.empty_like(x) for _ in range(3))
+    ext = ops._load_extension()
+
+    def microseconds(call):
+        times = []
+        for _ in range(5):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(50):
+                call()
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b) * 20)
+        return min(times)
+
+    for call in (lambda: ext.fullscan_forward_cl(g, x, out, False),
+                 lambda: ext.fullscan_backward_cl(g, out, go, gg, gx)):
+        automatic = microseconds(call)
+        ops.set_tiling(1)
+        try:
+            one_pass = microseconds(call)
+        finally:
+            ops.set_tiling(0)
+        assert automatic < 1.5 * one_pass
+
+
 @pytest.mark.parametrize("dtype", DTYPES, ids=str)
 @pytest.mark.parametrize("shape", [(1, 20000, 8), (2, 5000, 33), (4, 2500, 96)], ids=str)
 def test_matches_oracle_is_deterministic_and_mirrored(dtype, shape):
