@@ -1494,9 +1494,17 @@ ClBlockPlan plan_cl_blocks(int64_t batch, int64_t seqlen, int64_t dim, int64_t s
   const int vec = cl_vec(size);
   const int64_t nv = (dim + vec - 1) / vec;
   t.shared = (stride_t * size) % 128 != 0;
-  // narrow rows off the lines: a panel holds the whole row, so that tiles are contiguous (f16
-  // (45, 12181, 240) backward 350 -> 294 us); otherwise panels of up to kClbCv vectors
-  t.npan = (int)(t.shared && nv <= kClbMaxCv ? 1 : (nv + kClbCv - 1) / kClbCv);
+  // Narrow rows off the lines: a panel holds the whole row, so that tiles are contiguous;
+  // otherwise panels of up to kClbCv vectors. From 17 vectors a panel leaves its tiles 64-120 steps
+  // of 256, and with a few chains the look-back over that many more tiles costs more than the
+  // lines save, in the forward (one output) up to more of them. Measured on MI355X, split ->
+  // whole (us): f16 (2, 79243, 248) forward 75 -> 168, backward 127 -> 181, bf16 (4, 156512, 208)
+  // 228 -> 327, 393 -> 390, (6, 10033, 200) 22 -> 29, 44 -> 40, f16 (32, 28840, 184) 245 -> 251, 458 ->
+  // 368, fp32 (31, 1766, 116) 22.5 -> 20.1, 40.0 -> 37.4; at 16 vectors and fewer whole rows are even
+  // or faster with any number of chains.
+  const bool whole = t.shared && nv <= kClbMaxCv &&
+                     (nv <= 16 || batch >= 64 || (batch >= 4 && (bwd || nv <= 20)));
+  t.npan = (int)(whole ? 1 : (nv + kClbCv - 1) / kClbCv);
   t.cv = (int)((nv + t.npan - 1) / t.npan);
   t.groups = kClbThreads / t.cv;
   t.chains = batch * t.npan;

@@ -64,6 +64,16 @@ def test_exact_on_integer_data(dtype, shape):
     assert bits_equal(gg.cpu(), torch.from_numpy(gg_ref).to(dtype))
 
 
+# off the lines, rows of 17 to 32 vectors: whole (from 4 sequences in the backward, 64 in the
+# forward, up to 20 vectors from 4 in both) and split
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("shape", [(1, 1500, 15), (1, 1500, 17), (3, 700, 31), (4, 700, 31),
+                                   (3, 500, 20 - 1), (4, 500, 20), (4, 500, 21), (63, 150, 29),
+                                   (64, 150, 29)], ids=str)
+def test_whole_and_split_rows(dtype, shape):
+    test_exact_on_integer_data(dtype, shape)
+
+
 # around the length from which a sequence within one tile takes a block: 32 steps (the backward 16),
 # more with many chains, 96 at most; chains of 8 vectors on the lines, of up to 8 off them
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
