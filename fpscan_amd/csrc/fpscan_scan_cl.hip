@@ -1480,13 +1480,23 @@ constexpr int64_t kClbMaxBytes = 1ll << 30;
 // The largest tensor whose gates and output the forward of a training step keeps (as for rows).
 constexpr int64_t kClKeepMaxBytes = 128ll << 20;
 
+// Off the lines with enough strips for the one pass, below the size from which that yields to
+// tiles: only rows that fill half of a strip's 64 lanes or less, in chains of several tiles.
+// Measured on MI355X, one pass -> blocks, forward + backward (us): f16 (3456, 1308, 24), 3 vectors,
+// 517 + 919 -> 158 + 284, (7724, 265, 72), 9, 281 + 515 -> 212 + 358, bf16 (2387, 265, 120), 15, 115 +
+// 210 -> 99 + 168, (2065, 567, 200), 25, 316 + 578 -> 307 + 521, but (3128, 107, 184), 23, 83 + 152 -> 91 +
+// 145, f16 (782, 187, 184) 36 + 64 -> 46 + 71; wider rows with a last tile that is half empty lose,
+// bf16 (512, 257, 520) 105 + 182 -> 127 + 213, (128, 257, 2056) 116 + 192 -> 125 + 205, and with full
+// tiles are even, (64, 512, 4104) 201 + 356 -> 201 + 357.
+constexpr int64_t kClbNarrow = 16;
+constexpr int64_t kClbNarrowSteps = 256;
+
 // Taken in the automatic mode where one pass per strip lacks strips, whatever the size when
 // the rows are off the lines, else below kClbMaxBytes. Off the lines (measured on MI355X,
 // forward + backward, scan_cl_tiles -> this kernel, us): f16 (45, 12181, 240) 239 + 451 -> 193 +
 // 294, bf16 (56, 10271, 360) 512 + 906 -> 323 + 552, (8, 16384, 776) 178 + 360 -> 144 + 249, (10,
-// 32768, 1032) 636 + 1301 -> 479 + 928. There also with enough strips, if a chain has several
-// tiles: bf16 (64, 512, 4104) one pass 204 + 364 -> 203 + 356; on the lines the one pass is the
-// faster one (fp32 (64, 256, 4096) 138 + 243 against 158 + 261).
+// 32768, 1032) 636 + 1301 -> 479 + 928. On the lines the one pass is the faster one with enough
+// strips (fp32 (64, 256, 4096) 138 + 243 against 158 + 261).
 ClBlockPlan plan_cl_blocks(int64_t batch, int64_t seqlen, int64_t dim, int64_t stride_t, int size,
                            int tiling, bool bwd) {
   ClBlockPlan t{};
@@ -1532,9 +1542,14 @@ ClBlockPlan plan_cl_blocks(int64_t batch, int64_t seqlen, int64_t dim, int64_t s
     if (seqlen < least) return t;
   }
   const bool enough_strips = batch * ((nv + 63) / 64) >= kClMinTasks;
-  if (t.shared ? enough_strips && t.nseg < 2
-               : enough_strips || batch * seqlen * dim * size >= kClbMaxBytes)
-    return t;
+  const int64_t bytes = batch * seqlen * dim * size;
+  if (!t.shared) {
+    if (enough_strips || bytes >= kClbMaxBytes) return t;
+  } else if (enough_strips) {
+    if (t.nseg < 2) return t;
+    const bool narrow = nv <= kClbNarrow || (nv <= kClbMaxCv && seqlen >= kClbNarrowSteps);
+    if (bytes < kClTiledMinBytes && !narrow) return t;
+  }
   t.use = true;
   t.bytes = t.nseg > 1 ? (size_t)words * sizeof(uint64_t) : 0;
   return t;

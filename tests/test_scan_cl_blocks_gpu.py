@@ -74,6 +74,15 @@ def test_whole_and_split_rows(dtype, shape):
     test_exact_on_integer_data(dtype, shape)
 
 
+# off the lines with 512 strips or more: blocks up to 16 vectors (2 tiles and 1), up to 32 from 256
+# steps, the one pass otherwise
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("shape", [(513, 130, 15), (512, 120, 15), (512, 255, 17), (512, 256, 17),
+                                   (512, 65, 31), (256, 257, 65)], ids=str)
+def test_enough_strips_off_the_lines(dtype, shape):
+    test_short_sequences(dtype, shape)
+
+
 # around the length from which a sequence within one tile takes a block: 32 steps (the backward 16),
 # more with many chains, 96 at most; chains of 8 vectors on the lines, of up to 8 off them
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
