@@ -1473,10 +1473,22 @@ struct ClBlockPlan {
 // chains, bf16 (2, 2048, 1024) 13.2 / 13.5; 128 chains, bf16 (8, 2048, 1024) 38.7 / 41.0 and (4,
 // 4096, 2048) 70.8 / 71.2, 256 chains, bf16 (16, 1024, 1024) 37.2 / 38.6.
 constexpr int64_t kClbFewChains = 48;
-// Rows on 128-byte lines go to scan_cl_tiles from this size per tensor: at 512 MiB, bf16 (4,
-// 65536, 1024), this kernel takes 290 + 480 us against 312 + 480, at 1 GiB, (8, 65536, 1024),
-// 572 + 965 against 567 + 925.
+// From these sizes per tensor scan_cl_tiles takes over. Rows on the 128-byte lines: from 1 GiB,
+// where both measured even on average, blocks -> tiles, forward + backward (us): fp32 (4, 65536,
+// 1024) 535 + 913 -> 539 + 901, (8, 16384, 2048) 565 + 931 -> 533 + 933, bf16 (32, 16384, 1024) 665 +
+// 959 -> 578 + 960, (1, 65536, 8192) 540 + 933 -> 569 + 896; at 768 MiB fp32 (3, 65536, 1024) 406 +
+// 697 -> 433 + 689, bf16 (6, 65536, 1024) 420 + 717 -> 432 + 714. The 2-byte backward with 17 to 127
+// chains, whose tiles of a chain follow one another without a gap: from 512 MiB, bf16 (21, 212468,
+// 64), 21 chains, 570 -> 533, f16 (1, 216176, 1344), 21, 582 -> 552, bf16 (17, 119363, 192), 51, 741 ->
+// 722, but 10 chains, f16 (2, 567543, 320), 751 -> 812, 627 chains, (209, 8545, 192), 650 -> 665.
 constexpr int64_t kClbMaxBytes = 1ll << 30;
+constexpr int64_t kClbMaxBytesHalfBwd = 512ll << 20;
+// Split rows that start on 64-byte lines, whose pieces share only every second 128-byte line: from
+// 192 MiB, blocks -> tiles: f16 (12, 41207, 480) 453 MiB 314 + 551 -> 291 + 533, fp32 (38, 1347, 1168)
+// 228 MiB 161 + 278 -> 143 + 251, (3, 17087, 1296) 170 + 294 -> 162 + 271, bf16 (8, 22199, 672) 157 +
+// 271 -> 154 + 261, but (12, 2870, 2976) 196 MiB 136 + 240 -> 140 + 243 and (4, 3964, 1184) 36 MiB 33 +
+// 53 -> 39 + 57.
+constexpr int64_t kClbMaxBytesHalfLines = 192ll << 20;
 // The largest tensor whose gates and output the forward of a training step keeps (as for rows).
 constexpr int64_t kClKeepMaxBytes = 128ll << 20;
 
@@ -1492,7 +1504,7 @@ constexpr int64_t kClbNarrow = 16;
 constexpr int64_t kClbNarrowSteps = 256;
 
 // Taken in the automatic mode where one pass per strip lacks strips, whatever the size when
-// the rows are off the lines, else below kClbMaxBytes. Off the lines (measured on MI355X,
+// the rows are off the 64-byte lines, else below the sizes above. Off the lines (measured on MI355X,
 // forward + backward, scan_cl_tiles -> this kernel, us): f16 (45, 12181, 240) 239 + 451 -> 193 +
 // 294, bf16 (56, 10271, 360) 512 + 906 -> 323 + 552, (8, 16384, 776) 178 + 360 -> 144 + 249, (10,
 // 32768, 1032) 636 + 1301 -> 479 + 928. On the lines the one pass is the faster one with enough
@@ -1544,7 +1556,10 @@ ClBlockPlan plan_cl_blocks(int64_t batch, int64_t seqlen, int64_t dim, int64_t s
   const bool enough_strips = batch * ((nv + 63) / 64) >= kClMinTasks;
   const int64_t bytes = batch * seqlen * dim * size;
   if (!t.shared) {
-    if (enough_strips || bytes >= kClbMaxBytes) return t;
+    const bool half_bwd = bwd && size == 2 && t.chains > 16 && t.chains < 128;
+    if (enough_strips || bytes >= (half_bwd ? kClbMaxBytesHalfBwd : kClbMaxBytes)) return t;
+  } else if (t.npan > 1 && (stride_t * size) % 64 == 0 && bytes >= kClbMaxBytesHalfLines) {
+    return t;
   } else if (enough_strips) {
     if (t.nseg < 2) return t;
     const bool narrow = nv <= kClbNarrow || (nv <= kClbMaxCv && seqlen >= kClbNarrowSteps);
