@@ -1231,16 +1231,21 @@ int run(const Args& a, void* workspace, size_t ws_bytes, hipStream_t stream) {
                      (Gp::kFused && kMode == kBwd && nsub >= 16 && nsub <= 32 && from16);
   if (eight) w = 8;
   // Rows of 8 sub-chunks in the forward and reverse from 16 to 256 MiB, and with the fused gates
-  // rows of 8 always and of 4 in the forward and reverse: half the waves, each with two
+  // from 8 MiB rows of 8 and, in the forward and reverse, of 4: half the waves, each with two
   // sub-chunks in flight, so that a CU holds more rows at once and their loads, scans and stores
   // overlap. Measured on MI355X (us, one round of w waves -> two of w / 2): bf16 (4, 1024, 4096)
   // forward 18.7 -> 17.7, fp32 (8, 1024, 2048) 34.1 -> 32.6, 128 MiB 65.4 -> 64.3, 256 MiB 125.8 ->
   // 125.3, but 512 MiB 260.4 -> 265.2 and at 4 MiB 5.5 -> 5.6; fused gates on rows of 8 forward /
   // backward 19.4 / 31.6 -> 18.5 / 30.8 at 32 MiB, 67.0 / 112.7 -> 64.7 / 107.9 at 128 MiB, 130.8 /
   // 224.6 -> 126.7 / 213.9 at 256 MiB, forward on rows of 4 19.8 -> 18.5 at 32 MiB and 133.8 ->
-  // 129.5 at 256 MiB (the backward there 1-2 % slower). The plain backward loses 2 % on rows of 8,
-  // and the plain forward is even on rows of 4 at 32 MiB and loses 3 % at 256 MiB.
-  if (Gp::kFused ? nsub == 8 || (nsub == 4 && kMode != kBwd)
+  // 129.5 at 256 MiB (the backward there 1-2 % slower). Fused gates on smaller tensors, where few
+  // rows share a CU anyway and the second sub-chunk only lengthens each: bf16 rows of 8 at 1 / 4 /
+  // 6 / 8 / 16 MiB, forward 2.97 / 4.20 / 5.13 / 6.28 / 10.2 -> 3.15 / 4.08 / 5.17 / 5.75 / 9.4, backward
+  // 4.15 / 6.19 / 7.72 / 9.93 / 17.2 -> 4.38 / 6.35 / 7.32 / 8.46 / 17.3, rows of 4, forward 2.71 / 4.08 /
+  // 5.02 / 6.27 / 10.0 -> 3.04 / 3.94 / 5.52 / 5.61 / 9.4; fp32 crosses at the same size. The plain
+  // backward loses 2 % on rows of 8, and the plain forward is even on rows of 4 at 32 MiB and loses
+  // 3 % at 256 MiB.
+  if (Gp::kFused ? kib >= (8 << 10) && (nsub == 8 || (nsub == 4 && kMode != kBwd))
                  : kMode != kBwd && nsub == 8 && from16 && kib <= (256 << 10))
     w = nsub / 2;
   int u_max = (w == 1 && kMode != kBwd) ? 4
