@@ -158,11 +158,9 @@ at::Tensor fullscan_forward_saved(const at::Tensor& Ax, const at::Tensor& Bx,
   return run_forward(Ax, Bx, out, false, true);
 }
 
-std::tuple<at::Tensor, at::Tensor> fullscan_backward(const at::Tensor& gates,
-                                                     const at::Tensor& out,
-                                                     const at::Tensor& grad_out,
-                                                     const at::Tensor& grad_gates,
-                                                     const at::Tensor& grad_tokens) {
+// The fused backward; `saved`: after run_forward with `saved` (fpscan_scan_bwd_saved).
+void run_backward(const at::Tensor& gates, const at::Tensor& out, const at::Tensor& grad_out,
+                  const at::Tensor& grad_gates, const at::Tensor& grad_tokens, bool saved) {
   check_input(gates, "gates");
   check_input(out, "out");
   check_input(grad_out, "grad_out");
@@ -173,7 +171,7 @@ std::tuple<at::Tensor, at::Tensor> fullscan_backward(const at::Tensor& gates,
   check_like(grad_gates, gates, "grad_gates", "gates");
   check_like(grad_tokens, gates, "grad_tokens", "gates");
   check_seqlen(gates.size(2));
-  if (gates.numel() == 0) return {grad_gates, grad_tokens};
+  if (gates.numel() == 0) return;
   check_no_alias({&grad_gates, &grad_tokens}, {&gates, &out, &grad_out}, "fullscan_backward");
 
   c10::hip::HIPGuardMasqueradingAsCUDA guard(gates.device());
@@ -182,12 +180,28 @@ std::tuple<at::Tensor, at::Tensor> fullscan_backward(const at::Tensor& gates,
   const size_t ws_bytes =
       fpscan_workspace_bytes(gates.size(0), gates.size(1), gates.size(2), dt, FPSCAN_OP_BWD);
   at::Tensor ws = workspace(ws_bytes, gates);
-  const int status = fpscan_scan_bwd(gates.data_ptr(), out.data_ptr(), grad_out.data_ptr(),
-                                     grad_gates.data_ptr(), grad_tokens.data_ptr(),
-                                     gates.size(0), gates.size(1), gates.size(2),
-                                     gates.size(1) * gates.size(2), gates.size(2), dt,
-                                     ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, stream);
-  check_status(status);
+  const auto entry = saved ? fpscan_scan_bwd_saved : fpscan_scan_bwd;
+  check_status(entry(gates.data_ptr(), out.data_ptr(), grad_out.data_ptr(), grad_gates.data_ptr(),
+                     grad_tokens.data_ptr(), gates.size(0), gates.size(1), gates.size(2),
+                     gates.size(1) * gates.size(2), gates.size(2), dt,
+                     ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, stream));
+}
+
+std::tuple<at::Tensor, at::Tensor> fullscan_backward(const at::Tensor& gates,
+                                                     const at::Tensor& out,
+                                                     const at::Tensor& grad_out,
+                                                     const at::Tensor& grad_gates,
+                                                     const at::Tensor& grad_tokens) {
+  run_backward(gates, out, grad_out, grad_gates, grad_tokens, false);
+  return {grad_gates, grad_tokens};
+}
+
+std::tuple<at::Tensor, at::Tensor> fullscan_backward_saved(const at::Tensor& gates,
+                                                           const at::Tensor& out,
+                                                           const at::Tensor& grad_out,
+                                                           const at::Tensor& grad_gates,
+                                                           const at::Tensor& grad_tokens) {
+  run_backward(gates, out, grad_out, grad_gates, grad_tokens, true);
   return {grad_gates, grad_tokens};
 }
 
@@ -211,7 +225,7 @@ struct PScanFunction : public torch::autograd::Function<PScanFunction> {
     const at::Tensor& out = saved[1];
     at::Tensor grad_gates = at::empty_like(gates);
     at::Tensor grad_tokens = at::empty_like(gates);
-    fullscan_backward(gates, out, grads[0].contiguous(), grad_gates, grad_tokens);
+    run_backward(gates, out, grads[0].contiguous(), grad_gates, grad_tokens, true);
     return {grad_gates, grad_tokens};
   }
 };
@@ -531,6 +545,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "fused backward of the forward scan: (grad_gates, grad_tokens) (HIP, gfx950)",
         pybind11::arg("gates"), pybind11::arg("out"), pybind11::arg("grad_out"),
         pybind11::arg("grad_gates"), pybind11::arg("grad_tokens"));
+  m.def("fullscan_backward_saved", &fullscan_backward_saved,
+        "fullscan_backward after fullscan_forward_saved: launched for gates and an output that "
+        "are still in the memory-side cache", pybind11::arg("gates"), pybind11::arg("out"),
+        pybind11::arg("grad_out"), pybind11::arg("grad_gates"), pybind11::arg("grad_tokens"));
   m.def("pscan", &pscan,
         "differentiable scan: the forward kernel, and the fused backward kernel under autograd",
         pybind11::arg("gates"), pybind11::arg("tokens"));

@@ -56,6 +56,9 @@ struct Args {
   int64_t stride_d;
   int32_t seqlen;
   int32_t contiguous;
+  // host only, backward: the gates and the forward output were left in the memory-side cache
+  // (fpscan_scan_fwd_saved)
+  int32_t after_saved;
   // fused softplus gates only: per-channel rate (dim floats) and, for the backward, one
   // partial sum of d loss / d rate per row (rows floats, may be null)
   const float* rate;
@@ -1216,17 +1219,21 @@ int run(const Args& a, void* workspace, size_t ws_bytes, hipStream_t stream) {
   // L8192 68.1 -> 64.8); fused-gate backward on rows of 16-32 sub-chunks at 16-256 MiB 11-25 %
   // (bf16 8192 rows of L8192 152.4 -> 117.4). Elsewhere 8 waves measured slower (2-9 % on
   // rows of 2-8 rounds at 128-256 MiB, up to 5 % below 16 MiB, where a call takes about 7 us)
-  // or even (the plain backward on rows of 16 at 128-256 MiB). The plain backward takes 8
-  // waves on rows of any length at 16-128 MiB: two rows a CU hide each other's ring fill and
-  // drain at the row's ends, which shows once its gates and forward output come out of the
-  // memory-side cache (a training step: bf16 (1, 1024, 65536) 171.0 -> 164.3 us, (1, 512, 65536)
-  // 90.1 -> 85.0, fp32 (4, 1024, 8192) 166.4 -> 161.8; alone it is within 1.5 % either way, and
-  // at 192 MiB 1-4 % slower).
+  // or even (the plain backward on rows of 16 at 128-256 MiB). After a saved forward the plain
+  // backward takes 8 waves on rows of any length at 16-128 MiB, from a row per CU: two rows a CU
+  // hide each other's ring fill and drain at the row's ends, which shows once the gates and the
+  // forward output come out of the memory-side cache, and costs up to 3 % if they do not.
+  // Measured on MI355X, 16 waves -> 8, a training step / a backward over the same operands / over
+  // three sets of operands in turn: bf16 rows of L65536 at 128 MiB 165.0 -> 164.4 / 120.2 -> 122.1 /
+  // 120.2 -> 122.4 us, at 96 MiB 125.4 -> 123.7 / 95.4 -> 98.0 / 94.7 -> 96.1, at 64 MiB 86.7 -> 84.9 /
+  // 58.8 -> 59.0 / 61.1 -> 61.1, L32768 at 128 MiB 169.0 -> 164.3 / 115.1 -> 116.7 / 116.6 -> 118.1,
+  // fp32 L16384 at 128 MiB 166.6 -> 163.0 / 114.1 -> 117.7 / 118.5 -> 118.2; 64 rows of fp32 L65536,
+  // 16 MiB, 51.9 -> 53.6 / 33.0 -> 34.5 / 34.0 -> 35.4.
   const int64_t kib = a.rows * nsub;  // tensor size: a sub-chunk is 1 KiB
   const bool from16 = kib >= (16 << 10);
   const bool eight = (nsub >= 16 && nsub <= 64 && from16 && kib <= (64 << 10)) ||
-                     (kMode == kBwd && !Gp::kFused && nsub >= 16 && from16 &&
-                      kib <= (128 << 10)) ||
+                     (kMode == kBwd && !Gp::kFused && a.after_saved && nsub >= 16 &&
+                      a.rows >= 256 && from16 && kib <= (128 << 10)) ||
                      (kMode != kBwd && nsub == 16 && from16) ||
                      (Gp::kFused && kMode == kBwd && nsub >= 16 && nsub <= 32 && from16);
   if (eight) w = 8;
@@ -1444,10 +1451,10 @@ int fpscan_scan_fwd_saved(const void* gates, const void* tokens, void* out, int6
                                    static_cast<hipStream_t>(stream));
 }
 
-int fpscan_scan_bwd(const void* gates, const void* out, const void* grad_out, void* grad_gates,
+static int backward(const void* gates, const void* out, const void* grad_out, void* grad_gates,
                     void* grad_tokens, int64_t batch, int64_t dim, int64_t seqlen,
-                    int64_t stride_b, int64_t stride_d, int dtype, void* workspace,
-                    size_t workspace_bytes, void* stream) {
+                    int64_t stride_b, int64_t stride_d, int dtype, bool after_saved,
+                    void* workspace, size_t workspace_bytes, void* stream) {
   Args a{};
   const int st = validate(batch, dim, seqlen, stride_b, stride_d, dtype, &a);
   if (st != FPSCAN_OK) return st;
@@ -1461,7 +1468,24 @@ int fpscan_scan_bwd(const void* gates, const void* out, const void* grad_out, vo
   a.in2 = out;
   a.out0 = grad_tokens;
   a.out1 = grad_gates;
+  a.after_saved = after_saved;
   return dispatch<kBwd>(dtype, a, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+int fpscan_scan_bwd(const void* gates, const void* out, const void* grad_out, void* grad_gates,
+                    void* grad_tokens, int64_t batch, int64_t dim, int64_t seqlen,
+                    int64_t stride_b, int64_t stride_d, int dtype, void* workspace,
+                    size_t workspace_bytes, void* stream) {
+  return backward(gates, out, grad_out, grad_gates, grad_tokens, batch, dim, seqlen, stride_b,
+                  stride_d, dtype, false, workspace, workspace_bytes, stream);
+}
+
+int fpscan_scan_bwd_saved(const void* gates, const void* out, const void* grad_out,
+                          void* grad_gates, void* grad_tokens, int64_t batch, int64_t dim,
+                          int64_t seqlen, int64_t stride_b, int64_t stride_d, int dtype,
+                          void* workspace, size_t workspace_bytes, void* stream) {
+  return backward(gates, out, grad_out, grad_gates, grad_tokens, batch, dim, seqlen, stride_b,
+                  stride_d, dtype, true, workspace, workspace_bytes, stream);
 }
 
 int fpscan_scan_fwd_noalloc(const void* gates, const void* tokens, void* out, int64_t batch,

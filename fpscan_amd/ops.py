@@ -105,9 +105,9 @@ class PScan(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output: torch.Tensor):
         gates, out = ctx.saved_tensors
-        grad_output = grad_output.contiguous()
-        grad_gates, grad_tokens = scan_backward(gates, out, grad_output)
-        return grad_gates, grad_tokens
+        grad_gates, grad_tokens = torch.empty_like(gates), torch.empty_like(gates)
+        return _load_extension().fullscan_backward_saved(gates, out, grad_output.contiguous(),
+                                                         grad_gates, grad_tokens)
 
 
 def pscan(gates: torch.Tensor, tokens: torch.Tensor) -> torch.Tensor:

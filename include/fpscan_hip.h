@@ -134,6 +134,16 @@ int fpscan_scan_bwd(const void* gates, const void* out, const void* grad_out,
                     int dtype,
                     void* workspace, size_t workspace_bytes, void* stream);
 
+/* fpscan_scan_bwd after fpscan_scan_fwd_saved of the same tensors: the same results up to the
+ * order of fp32 products and the same workspace, with the launch that suits operands still in the
+ * memory-side cache. */
+int fpscan_scan_bwd_saved(const void* gates, const void* out, const void* grad_out,
+                          void* grad_gates, void* grad_tokens,
+                          int64_t batch, int64_t dim, int64_t seqlen,
+                          int64_t stride_b, int64_t stride_d,
+                          int dtype,
+                          void* workspace, size_t workspace_bytes, void* stream);
+
 /* Device workspace, in bytes, that the tiled path of fpscan_scan_fwd (op FPSCAN_OP_FWD) or
  * fpscan_scan_bwd (FPSCAN_OP_BWD) uses for this problem; 0 when the problem takes the
  * row-streaming path (which needs none). The two can differ: the backward tiles from a

@@ -8,7 +8,8 @@ import torch
 from torch.profiler import ProfilerActivity, profile
 
 import fpscan_amd
-from scan_helpers import DEVICE
+import oracle
+from scan_helpers import DEVICE, check
 
 pytestmark = [
     pytest.mark.gpu,
@@ -44,3 +45,29 @@ def test_waves_of_softplus_rows_of_four_and_eight_sub_chunks(dtype, subs, mib, f
         assert (name, args[2]) == ("scan_long_rows", str(fwd_waves))
     (name, args), = kernels(lambda: fpscan_amd.scan_backward_softplus(z, rate, z, z))
     assert (name, args[2]) == ("scan_long_rows", str(bwd_waves))
+
+
+# the backward takes 8 waves on rows of any length from 16 to 128 MiB after a saved forward, from 256
+# rows; on its own only on rows of 16 to 64 sub-chunks up to 64 MiB (a sub-chunk is 1 KiB)
+@pytest.mark.parametrize("rows,subs,alone,after", [(256, 128, 16, 8), (255, 128, 16, 16),
+                                                   (1024, 128, 16, 8), (1025, 128, 16, 16),
+                                                   (1024, 16, 8, 8), (1023, 16, 16, 16),
+                                                   (4096, 32, 16, 8)], ids=str)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+def test_waves_of_the_backward(dtype, rows, subs, alone, after):
+    shape = (1, rows, subs * (1024 // torch.empty((), dtype=dtype).element_size()))
+    g = torch.sigmoid(3 + torch.randn(shape, device=DEVICE)).to(dtype)
+    x, go = (torch.randn(shape, device=DEVICE).to(dtype) for _ in range(2))
+    y = fpscan_amd.scan_forward(g, x)
+    (name, args), = kernels(lambda: fpscan_amd.scan_backward(g, y, go))
+    assert (name, args[2]) == ("scan_long_rows", str(alone))
+    for apply in (fpscan_amd.pscan, fpscan_amd.PScan.apply):
+        leaves = [t.clone().requires_grad_() for t in (g, x)]
+        out = apply(*leaves)
+        (name, args), = kernels(lambda: out.backward(go))
+        assert (name, args[2]) == ("scan_long_rows", str(after))
+        pick = [0, rows - 1]
+        gg_ref, gx_ref = oracle.scan_bwd_f64(g[:, pick].cpu(), out[:, pick].detach().cpu(),
+                                             go[:, pick].cpu())
+        check(leaves[0].grad[:, pick].cpu(), gg_ref, dtype, "grad_gates")
+        check(leaves[1].grad[:, pick].cpu(), gx_ref, dtype, "grad_tokens")
