@@ -205,6 +205,15 @@ std::tuple<at::Tensor, at::Tensor> fullscan_backward_saved(const at::Tensor& gat
   return {grad_gates, grad_tokens};
 }
 
+// Whether autograd records a call on these tensors: the forward of a training step, not of an
+// evaluation of the same parameters under no_grad. (Inside forward() grad mode is off.)
+bool backward_follows(std::initializer_list<at::Tensor> inputs) {
+  if (!at::GradMode::is_enabled()) return false;
+  for (const at::Tensor& t : inputs)
+    if (t.requires_grad()) return true;
+  return false;
+}
+
 // ---- pscan as an autograd function in C++: the same computation as the Python PScan
 // (fpscan/ops.py:61-87: the forward saves (gates, out), the backward hands grad_output to the
 // fused backward), with the forward and backward entered from the autograd engine without a
@@ -212,9 +221,9 @@ std::tuple<at::Tensor, at::Tensor> fullscan_backward_saved(const at::Tensor& gat
 // host time per step.
 struct PScanFunction : public torch::autograd::Function<PScanFunction> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& gates,
-                            const at::Tensor& tokens) {
+                            const at::Tensor& tokens, bool saved) {
     at::Tensor out = at::empty_like(tokens);
-    run_forward(gates, tokens, out, false, gates.requires_grad() || tokens.requires_grad());
+    run_forward(gates, tokens, out, false, saved);
     ctx->save_for_backward({gates, out});
     return out;
   }
@@ -226,12 +235,12 @@ struct PScanFunction : public torch::autograd::Function<PScanFunction> {
     at::Tensor grad_gates = at::empty_like(gates);
     at::Tensor grad_tokens = at::empty_like(gates);
     run_backward(gates, out, grads[0].contiguous(), grad_gates, grad_tokens, true);
-    return {grad_gates, grad_tokens};
+    return {grad_gates, grad_tokens, at::Tensor()};
   }
 };
 
 at::Tensor pscan(const at::Tensor& gates, const at::Tensor& tokens) {
-  return PScanFunction::apply(gates, tokens);
+  return PScanFunction::apply(gates, tokens, backward_follows({gates, tokens}));
 }
 
 // ---- channel-last (batch, seqlen, dim): no reference counterpart (README.md:94-99 has
@@ -319,9 +328,9 @@ std::tuple<at::Tensor, at::Tensor> fullscan_backward_cl(const at::Tensor& gates,
 // The channel-last scan as an autograd function in C++ (see PScanFunction).
 struct PScanClFunction : public torch::autograd::Function<PScanClFunction> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& gates,
-                            const at::Tensor& tokens) {
+                            const at::Tensor& tokens, bool saved) {
     at::Tensor out = at::empty_like(tokens);
-    run_forward_cl(gates, tokens, out, false, gates.requires_grad() || tokens.requires_grad());
+    run_forward_cl(gates, tokens, out, false, saved);
     ctx->save_for_backward({gates, out});
     return out;
   }
@@ -333,12 +342,12 @@ struct PScanClFunction : public torch::autograd::Function<PScanClFunction> {
     at::Tensor grad_gates = at::empty_like(gates);
     at::Tensor grad_tokens = at::empty_like(gates);
     fullscan_backward_cl(gates, out, grads[0].contiguous(), grad_gates, grad_tokens);
-    return {grad_gates, grad_tokens};
+    return {grad_gates, grad_tokens, at::Tensor()};
   }
 };
 
 at::Tensor pscan_cl(const at::Tensor& gates, const at::Tensor& tokens) {
-  return PScanClFunction::apply(gates, tokens);
+  return PScanClFunction::apply(gates, tokens, backward_follows({gates, tokens}));
 }
 
 // ---- dimwise_forward: csrc/main.cpp:10, csrc/dimwise/dimwise.h:27-42 (CHECK_INPUT on all
@@ -495,10 +504,9 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> softplus_gradients(const at::Tens
 // The softplus-gate scan as an autograd function in C++ (see PScanFunction).
 struct PScanSoftplusFunction : public torch::autograd::Function<PScanSoftplusFunction> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& z,
-                            const at::Tensor& rate, const at::Tensor& tokens) {
+                            const at::Tensor& rate, const at::Tensor& tokens, bool saved) {
     at::Tensor out = at::empty_like(tokens);
-    run_forward_softplus(z, rate, tokens, out, false,
-                         z.requires_grad() || rate.requires_grad() || tokens.requires_grad());
+    run_forward_softplus(z, rate, tokens, out, false, saved);
     ctx->save_for_backward({z, rate, out});
     return out;
   }
@@ -507,12 +515,12 @@ struct PScanSoftplusFunction : public torch::autograd::Function<PScanSoftplusFun
     const auto saved = ctx->get_saved_variables();
     auto [grad_z, grad_rate, grad_tokens] =
         softplus_gradients(saved[0], saved[1], saved[2], grads[0].contiguous());
-    return {grad_z, grad_rate, grad_tokens};
+    return {grad_z, grad_rate, grad_tokens, at::Tensor()};
   }
 };
 
 at::Tensor pscan_softplus(const at::Tensor& z, const at::Tensor& rate, const at::Tensor& tokens) {
-  return PScanSoftplusFunction::apply(z, rate, tokens);
+  return PScanSoftplusFunction::apply(z, rate, tokens, backward_follows({z, rate, tokens}));
 }
 
 // Look-back waits that gave up on the tensors' device since the library was loaded (waits for

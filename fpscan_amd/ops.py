@@ -16,7 +16,9 @@ Drop-in for ``fpscan/ops.py`` of saeeddhqan/fpscan:
   Python call in the forward and in the backward. ``PScan.apply`` keeps working.
   ``pscan_channel_last`` and ``pscan_softplus`` have C++ twins likewise.
 * The autograd forwards call the extension's ``*_saved`` forms: the same results, with the
-  gates and the output left in the memory-side cache for the backward while they fit.
+  gates and the output left in the memory-side cache for the backward while they fit. The C++
+  functions do so only where autograd records the call; the Python classes, whose ``forward``
+  cannot see that, always.
 """
 from __future__ import annotations
 

@@ -71,3 +71,24 @@ def test_waves_of_the_backward(dtype, rows, subs, alone, after):
                                              go[:, pick].cpu())
         check(leaves[0].grad[:, pick].cpu(), gg_ref, dtype, "grad_gates")
         check(leaves[1].grad[:, pick].cpu(), gx_ref, dtype, "grad_tokens")
+
+
+# the last template argument of scan_long_rows and scan_cl_blocks is the cache policy, 0 if streamed
+@pytest.mark.parametrize("name,shape", [("pscan", (2, 64, 4096)), ("pscan_channel_last", (2, 2048, 256)),
+                                        ("pscan_softplus", (2, 64, 4096))])
+def test_a_forward_that_autograd_does_not_record_streams(name, shape):
+    make = lambda *s: torch.rand(s, device=DEVICE, requires_grad=True)  # noqa: E731
+    inputs = [make(*shape), make(*shape)]
+    if name == "pscan_softplus":
+        inputs.insert(1, make(shape[1]))
+    call = getattr(fpscan_amd, name)
+    policy = lambda f: kernels(f)[-1][1][-1]  # noqa: E731
+    assert policy(lambda: call(*inputs)) != "0"
+    with torch.no_grad():
+        assert policy(lambda: call(*inputs)) == "0"
+        assert not call(*inputs).requires_grad
+    plain = [t.detach() for t in inputs]
+    assert policy(lambda: call(*plain)) == "0"
+    for i in range(len(inputs)):  # any one of them is enough
+        one = [t.requires_grad_() if i == j else t for j, t in enumerate(t.detach() for t in inputs)]
+        assert policy(lambda: call(*one)) != "0"
