@@ -883,7 +883,7 @@ scan_cl_tiles(const ClArgs a, uint64_t* __restrict__ status, const int64_t ntile
 // measured 2-10 % slower, wider ones more. K = 8 aggregates: 16 take 32 registers more (and
 // spill at R = 8), 1-3 % slower; 4 lose 8 % with few chains. The forward takes R = 8 (256 steps
 // a tile; 4 measured up to 20 % slower with few chains, even otherwise), the backward R = 4,
-// or 8 below kClbFewChains, where the look-back's latency bounds it (see plan_cl_blocks).
+// or 8 where the look-back bounds it or one tile then holds the sequence (see kClbLongTiles).
 //
 // Cache policies (kPol): streamed; kClbSaved, the forward of a training step (gates and
 // output left in the memory-side cache, see kKeepBoth); kClbShared, rows that do not start on
@@ -1468,11 +1468,21 @@ struct ClBlockPlan {
                  // and claim counters; 0 with one tile per chain
 };
 
-// The backward takes R = 8 below this many chains. Measured on MI355X, R = 4 against 8 (us):
-// 16 chains, bf16 (1, 65536, 1024) 143.0 / 135.8, 39 chains, f16 (3, 1000, 776) 17.3 / 13.9; 32
-// chains, bf16 (2, 2048, 1024) 13.2 / 13.5; 128 chains, bf16 (8, 2048, 1024) 38.7 / 41.0 and (4,
-// 4096, 2048) 70.8 / 71.2, 256 chains, bf16 (16, 1024, 1024) 37.2 / 38.6.
-constexpr int64_t kClbFewChains = 48;
+// The backward on the lines takes R = 4, whose tiles need fewer registers, except
+// - where one tile of R = 8 holds a sequence that takes two of R = 4: no status, no look-back. Measured
+//   on MI355X, R = 4 -> 8 (us): bf16 (2, 200, 256), 8 chains, 8.5 -> 5.3, (2, 256, 8192), 256, 11.8 ->
+//   8.1, fp32 (2, 130, 2048), 128, 9.0 -> 5.0, (2, 256, 6400), 400, 17.4 -> 15.8, (8, 130, 12000), 3000,
+//   65.5 -> 43.8;
+// - from this many tiles per chain with fewer than this many chains, where the look-back bounds the
+//   call: bf16 (2, 4096, 1408), 44 chains, 31.1 -> 28.5, (2, 8192, 1728), 54, 64.5 -> 59.8, (2, 32768,
+//   2240), 70, 297 -> 276, (2, 32768, 3200), 100, 399 -> 387, (2, 250000, 64), 2, 224 -> 132, fp32 (1,
+//   8192, 1504), 47, 55.5 -> 50.7, but 128 chains, (2, 8192, 2048), 119.0 -> 120.3.
+// With fewer tiles R = 4 is the faster one, bf16 (2, 1000, 1024), 32 chains, 10.4 -> 11.5, fp32 (2,
+// 2048, 704), 44, 17.8 -> 20.0, bf16 (2, 2048, 1664), 52, 20.1 -> 20.6; around 12 tiles that holds up to
+// 30 chains, bf16 (2, 3000, 256), 8, 11.5 -> 11.3, (1, 3000, 960), 15, 15.1 -> 17.2, fp32 (2, 3000, 480),
+// 30, 18.6 -> 20.2, (1, 3000, 2016), 63, 31.9 -> 27.2, bf16 (2, 3000, 1408), 44, 23.8 -> 22.4.
+constexpr int64_t kClbLongTiles = 12;
+constexpr int64_t kClbManyChains = 128;
 // From these sizes per tensor scan_cl_tiles takes over. Rows on the 128-byte lines: from 1 GiB,
 // where both measured even on average, blocks -> tiles, forward + backward (us): fp32 (4, 65536,
 // 1024) 535 + 913 -> 539 + 901, (8, 16384, 2048) 565 + 931 -> 533 + 933, bf16 (32, 16384, 1024) 665 +
@@ -1530,7 +1540,10 @@ ClBlockPlan plan_cl_blocks(int64_t batch, int64_t seqlen, int64_t dim, int64_t s
   t.cv = (int)((nv + t.npan - 1) / t.npan);
   t.groups = kClbThreads / t.cv;
   t.chains = batch * t.npan;
-  t.r = bwd && !t.shared && t.chains >= kClbFewChains ? 4 : 8;
+  const int64_t steps8 = 8 * (int64_t)t.groups;
+  const bool one_tile = seqlen <= steps8 && 2 * seqlen > steps8;
+  const bool long_chains = seqlen >= kClbLongTiles * steps8 && t.chains < kClbManyChains;
+  t.r = bwd && !t.shared && !one_tile && !long_chains ? 4 : 8;
   const int64_t steps = (int64_t)t.groups * t.r;
   if (seqlen > INT32_MAX - steps) return t;  // the last tile's end stays within 32 bits
   t.nseg = (seqlen + steps - 1) / steps;

@@ -92,3 +92,25 @@ def test_a_forward_that_autograd_does_not_record_streams(name, shape):
     for i in range(len(inputs)):  # any one of them is enough
         one = [t.requires_grad_() if i == j else t for j, t in enumerate(t.detach() for t in inputs)]
         assert policy(lambda: call(*one)) != "0"
+
+
+# scan_cl_blocks<type, mode, steps a lane, cache policy>: the backward on the 128-byte lines (chains of
+# 8 vectors) takes 8 steps a lane where one tile of 256 steps holds a sequence of more than 128, and
+# from 12 such tiles below 128 chains
+@pytest.mark.parametrize("seqlen,chains,steps", [(128, 3, 4), (129, 3, 8), (256, 3, 8), (257, 3, 4),
+                                                 (128, 60, 4), (256, 60, 8), (257, 60, 4),
+                                                 (3071, 20, 4), (3072, 20, 8), (3072, 127, 8),
+                                                 (3072, 128, 4)], ids=str)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+def test_steps_of_the_channel_last_backward(dtype, seqlen, chains, steps):
+    shape = (1, seqlen, chains * 128 // torch.empty((), dtype=dtype).element_size())
+    g = (0.9 + 0.09 * torch.rand(shape, device=DEVICE)).to(dtype)
+    y, go = (torch.randn(shape, device=DEVICE).to(dtype) for _ in range(2))
+    run = lambda: fpscan_amd.scan_backward_channel_last(g, y, go)  # noqa: E731
+    name, args = kernels(run)[-1]
+    assert (name, args[2]) == ("scan_cl_blocks", str(steps))
+    gg, gx = run()
+    pick = [0, 1, shape[2] - 1]
+    gg_ref, gx_ref = oracle.scan_bwd_f64_channel_last(*(t[..., pick].cpu() for t in (g, y, go)))
+    check(gx[..., pick].cpu(), gx_ref, dtype, "grad_tokens")
+    check(gg[..., pick].cpu(), gg_ref, dtype, "grad_gates")
