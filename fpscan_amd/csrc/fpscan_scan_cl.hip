@@ -1583,9 +1583,12 @@ ClBlockPlan plan_cl_blocks(int64_t batch, int64_t seqlen, int64_t dim, int64_t s
   return t;
 }
 
+// Rows off the lines always take R = 8 (see plan_cl_blocks).
 template <class E, int kMode, int R>
 const void* cl_blocks_kernel(bool shared, bool saved) {
-  if (shared) return reinterpret_cast<const void*>(&scan_cl_blocks<E, kMode, R, kClbShared>);
+  if constexpr (R == 8) {
+    if (shared) return reinterpret_cast<const void*>(&scan_cl_blocks<E, kMode, R, kClbShared>);
+  }
   if constexpr (kMode == kFwd) {
     if (saved) return reinterpret_cast<const void*>(&scan_cl_blocks<E, kMode, R, kClbSaved>);
   }
@@ -1801,7 +1804,8 @@ size_t fpscan_workspace_bytes_cl(int64_t batch, int64_t seqlen, int64_t dim, int
   const ClTilePlan tiles =
       plan_cl_tiles(batch, seqlen, dim, stride_t, size, fpscan_detail::tiling_mode());
   // the block path's words fit into the tiled path's almost always (off the lines its tiles
-  // can be shorter); the larger of the two serves both
+  // can be shorter); the larger of the two serves both, also where blocks need none (one tile a
+  // chain), so that the size of a problem stays what it is without the block path
   const size_t other =
       tiles.use ? tiles.bytes : plan_cl(batch, seqlen, dim, stride_t, size).bytes;
   return blocks.use && blocks.bytes > other ? blocks.bytes : other;
