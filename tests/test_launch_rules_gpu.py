@@ -6,7 +6,7 @@ import torch
 
 import fpscan_amd
 import oracle
-from scan_helpers import DEVICE, check
+from scan_helpers import DEVICE, NORM_TOL, check
 
 pytestmark = [
     pytest.mark.gpu,
@@ -50,6 +50,7 @@ def test_softplus_rows_of_four_and_eight_sub_chunks(dtype, rows, subs, reverse):
         gz_ref, gr_ref, gx_ref = oracle.scan_bwd_softplus_f64(at[0], r, y[:, pick].cpu(), at[2])
         check(gz[:, pick].cpu(), gz_ref, dtype, "grad_z")
         check(gx[:, pick].cpu(), gx_ref, dtype, "grad_tokens")
+        assert oracle.normwise_error(gr[pick], gr_ref) <= max(NORM_TOL[dtype], 1e-4)  # as test_softplus
 
 
 # short rows (64 elements): one wave per block from 64 MiB per tensor, a last block that is
@@ -60,6 +61,33 @@ def test_softplus_rows_of_four_and_eight_sub_chunks(dtype, rows, subs, reverse):
                                         (torch.bfloat16, (1 << 19) + 5)], ids=str)
 def test_short_rows_around_64_mib(dtype, rows):
     _check(dtype, rows, 64 * torch.empty((), dtype=dtype).element_size() / 1024)
+
+
+# the same kernels with the fused gates, and the plain reverse: the fewest and the most lanes a row (4 and
+# 32; fp32 8), rows that leave the last block (16 to 2 rows) partly empty, just below 64 MiB and above
+@pytest.mark.parametrize("below", [True, False], ids=["below", "above"])
+@pytest.mark.parametrize("dtype,L", [(torch.bfloat16, 32), (torch.float16, 32), (torch.float16, 256),
+                                     (torch.float32, 32), (torch.float32, 128)], ids=str)
+def test_short_rows_with_fused_gates_and_reverse(dtype, L, below):
+    rows = (64 << 20) // (L * torch.empty((), dtype=dtype).element_size()) + (-1 if below else 3)
+    gen = torch.Generator(device=DEVICE).manual_seed(rows)
+    z, x, go = (torch.randn((1, rows, L), generator=gen, device=DEVICE).to(dtype) for _ in range(3))
+    rate = 0.1 * torch.rand(rows, generator=gen, device=DEVICE)
+    pick = torch.tensor(sorted({0, 1, rows // 2, *range(rows - 17, rows)}))
+    zp, xp, gop, rp = *(t[:, pick].cpu() for t in (z, x, go)), rate[pick].cpu()
+    for reverse in (True, False):
+        y = fpscan_amd.scan_forward_softplus(z, rate, x, reverse)
+        check(y[:, pick].cpu(), oracle.scan_softplus_f64(zp, rp, xp, reverse), dtype, "softplus")
+        assert torch.isfinite(y).all()
+    gz, gr, gx = fpscan_amd.scan_backward_softplus(z, rate, y, go)
+    gz_ref, gr_ref, gx_ref = oracle.scan_bwd_softplus_f64(zp, rp, y[:, pick].cpu(), gop)
+    check(gz[:, pick].cpu(), gz_ref, dtype, "grad_z")
+    check(gx[:, pick].cpu(), gx_ref, dtype, "grad_tokens")
+    assert oracle.normwise_error(gr[pick], gr_ref) <= max(NORM_TOL[dtype], 1e-4)  # as test_softplus
+    assert all(torch.isfinite(t).all() for t in (gz, gr, gx))
+    y = fpscan_amd.scan_forward(torch.sigmoid(3 + z), x, reverse=True)
+    check(y[:, pick].cpu(), oracle.scan_f64(torch.sigmoid(3 + z)[:, pick].cpu(), xp, True), dtype,
+          "reverse")
 
 
 def _check(dtype, rows, subs):
