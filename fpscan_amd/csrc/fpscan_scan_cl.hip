@@ -864,7 +864,9 @@ scan_cl_tiles(const ClArgs a, uint64_t* __restrict__ status, const int64_t ntile
 // tell: a carry whose composition is not finite is replaced by the predecessor's end value, and
 // a column whose state leaves the range inside the tile has the values entering its groups
 // computed again, one step after the other. So every value is what the serial recurrence gives
-// wherever the products over one lane's R steps are finite. Every tile publishes its end value
+// wherever the products over one lane's R steps are finite, up to one case: where a state itself
+// overflows and a tile's product of gates brings it back, the tiles that follow hold the finite
+// value that the product gives, not the Inf or NaN of the steps. Every tile publishes its end value
 // (a composed one that is not finite only once it is settled); a NaN in it is passed on at
 // once, as it makes every later state of its chain NaN in the recurrence too. Only chains with
 // such values pay, by waiting for one tile after the other: bf16 (1, 65536, 1024) 86 -> 384 us

@@ -115,9 +115,11 @@ int fpscan_scan_fwd_noalloc(const void* gates, const void* tokens, void* out,
                             int dtype, int reverse, void* stream);
 
 /* The forward of a training step: fpscan_scan_fwd's forward direction, with the same results,
- * for a caller that will hand `gates` and `out` to fpscan_scan_bwd. Up to 128 MiB per tensor it
- * reads the gates and writes the output with the cache policy that leaves them in the 256 MiB
- * memory-side cache instead of streaming them past it. Same workspace as fpscan_scan_fwd. */
+ * for a caller that will hand `gates` and `out` to fpscan_scan_bwd_saved. Up to 128 MiB per tensor
+ * it reads the gates and writes the output with the cache policy that leaves them in the 256 MiB
+ * memory-side cache instead of streaming them past it: rows of at least 1 KiB, and shorter ones
+ * from 64 MiB. Below, those load with that policy in every forward and stream the output. Same
+ * workspace as fpscan_scan_fwd. */
 int fpscan_scan_fwd_saved(const void* gates, const void* tokens, void* out,
                           int64_t batch, int64_t dim, int64_t seqlen,
                           int64_t stride_b, int64_t stride_d, int dtype,
@@ -158,14 +160,21 @@ size_t fpscan_workspace_bytes(int64_t batch, int64_t dim, int64_t seqlen, int dt
  * Same semantics as fpscan_scan_fwd on the transposed data (first gate ignored, zero initial
  * state, fp32 arithmetic), without the transposes. Any seqlen >= 1; dim, stride_t and
  * stride_b multiples of 16/itemsize elements; pointers 16-byte aligned; `out` may alias
- * `tokens` or `gates` exactly. With at least 512 strips of 64 16-byte vectors
- * (batch * dim / (64 * 16/itemsize)) and less than 512 MiB per tensor, one wave scans each
- * strip in one pass. Otherwise the time axis is tiled and needs fpscan_workspace_bytes_cl()
- * bytes of workspace: a single pass whose tiles (64 columns by 128 steps, 64 in fp32) look
- * back along time (3 N s bytes forward, results independent of timing). Where a tile does
- * not apply (seqlen within one tile, or a tile's rows beyond a 2 GiB buffer range), fewer
- * than 512 strips take segments (aggregates, carries, then the segments again: 5 N s bytes)
- * and more take the one pass. Without the workspace the call runs one pass per strip
+ * `tokens` or `gates` exactly. Four paths, in this order:
+ * - blocks: one pass (3 N s bytes forward) of tiles of one to 32 16-byte vectors by 32 to 2048
+ *   steps (8 vectors by 128 or 256 on whole 128-byte rows) that look back along time. With fewer
+ *   than 512 strips of 64 16-byte vectors (batch * ceil(dim / (64 * 16/itemsize))) below 1 GiB per
+ *   tensor (512 MiB in the 2-byte backward with 17 to 127 panels), except sequences of a few
+ *   steps; and where rows (stride_t * itemsize) are not whole 128-byte lines at any size, but for
+ *   rows on 64-byte lines of several panels from 192 MiB, and with 512 strips or more
+ *   below 512 MiB only on narrow rows (16 vectors, 32 from 256 steps). A sequence within one tile
+ *   uses no workspace.
+ * - tiles of 64 columns by 128 steps (64 in fp32) with a look-back, on a persistent grid: fewer
+ *   than 512 strips, or 512 MiB and more per tensor, if seqlen is more than one tile.
+ * - fewer than 512 strips: segments (aggregates, carries, then the segments again: 5 N s bytes).
+ * - one wave per strip in one pass.
+ * The first three need fpscan_workspace_bytes_cl() bytes of workspace; results do not depend on
+ * timing. With less the call takes the next path that it suffices for, at last the one pass
  * (correct, slower), except that a batch slab of more than about 2 GiB needs the workspace
  * (FPSCAN_ERR_WORKSPACE otherwise). Calls sharing a workspace must not overlap.
  * No reference counterpart: the reference supports (batch, dim, seqlen) only and tells callers
@@ -177,7 +186,9 @@ int fpscan_scan_fwd_cl(const void* gates, const void* tokens, void* out,
                        void* workspace, size_t workspace_bytes, void* stream);
 
 /* fpscan_scan_fwd_cl's forward direction for a caller that will hand `gates` and `out` to
- * fpscan_scan_bwd_cl (see fpscan_scan_fwd_saved): the same results and workspace. */
+ * fpscan_scan_bwd_cl (see fpscan_scan_fwd_saved): the same results and workspace. Calls that take
+ * blocks keep gates and output up to 128 MiB per tensor; the other paths stream, as
+ * fpscan_scan_fwd_cl does. */
 int fpscan_scan_fwd_cl_saved(const void* gates, const void* tokens, void* out,
                              int64_t batch, int64_t seqlen, int64_t dim,
                              int64_t stride_b, int64_t stride_t, int dtype,
@@ -197,7 +208,8 @@ int fpscan_scan_bwd_cl(const void* gates, const void* out, const void* grad_out,
 
 /* Workspace, in bytes, for the path with a look-back (tiles or blocks) or the segments that
  * this problem takes (0: one pass per strip); it depends on fpscan_set_tiling's setting and can
- * differ between the operations. */
+ * differ between the operations. Never less than what the problem takes without blocks, also where
+ * a block path with one tile per sequence uses none. */
 size_t fpscan_workspace_bytes_cl(int64_t batch, int64_t seqlen, int64_t dim, int64_t stride_t,
                                  int dtype, int op);
 
