@@ -1542,6 +1542,22 @@ ClBlockPlan plan_cl_blocks(int64_t batch, int64_t seqlen, int64_t dim, int64_t s
   t.cv = (int)((nv + t.npan - 1) / t.npan);
   t.groups = kClbThreads / t.cv;
   t.chains = batch * t.npan;
+  // Rows of 1 to 3 vectors would have tiles of 2048 to 680 steps, in which one thread a column
+  // composes 256 to 85 maps, twice: the call's latency where a chain has several tiles. Those take
+  // 64 groups (512 steps) while all tiles are resident at once, else 128 at most. Measured on
+  // MI355X, scan_cl_tiles / every thread in a group -> this, forward (us): bf16 (4, 4500, 8) 16.6 /
+  // 22.4 -> 14.6, (4, 2000, 16) 14.5 / 16.8 -> 14.1, (64, 4500, 8) 34.9 / 22.6 -> 13.6, fp32 (4, 2600,
+  // 4) 18.3 / 21.8 -> 13.6, and with 128 groups (200, 10000, 8) 146 / 42.6 -> 38.5 (64: 43.5), fp32
+  // (500, 4500, 4) 265 / 53.6 -> 46.0 (64: 48.8). Chains of more than 32 such tiles are even, (1,
+  // 40000, 8) 18.1 (128: 17.9), (1, 40000, 24) 17.8 -> 19.0.
+  if (t.groups > 64 && seqlen > 8 * (int64_t)t.groups) {
+    const int64_t tiles64 = (seqlen + 511) / 512;
+    const int64_t resident = 256 * (bwd ? 3 : 4);  // workgroups of R = 8, see scan_cl_blocks
+    if (tiles64 <= 32 && t.chains * tiles64 <= resident)
+      t.groups = 64;
+    else if (t.groups > 128)
+      t.groups = 128;
+  }
   const int64_t steps8 = 8 * (int64_t)t.groups;
   const bool one_tile = seqlen <= steps8 && 2 * seqlen > steps8;
   const bool long_chains = seqlen >= kClbLongTiles * steps8 && t.chains < kClbManyChains;

@@ -23,7 +23,7 @@ pytestmark = [
 # (batch, seqlen, 16-byte vectors per row): on the lines, 8 vectors = 32 groups: tiles of 256
 # steps (8 per lane), of 128 in the backward from 48 chains; one tile exactly, one step less
 # and more; 11 tiles (an end value two look-backs back); off the lines, whole rows as panels
-# (1, 2, 9, 31 vectors: 256, 128, 28, 8 groups) and split ones (33 -> 5 panels of 7); 2 batches of
+# (1, 2, 9, 31 vectors: 64, 64, 28, 8 groups) and split ones (33 -> 5 panels of 7); 2 batches of
 # 24 panels: the backward's shorter tiles
 SHAPES = [(1, 255, 8), (2, 256, 8), (1, 257, 8), (1, 2600, 8), (3, 300, 16), (2, 2049, 1),
           (1, 4500, 2), (2, 3000, 9), (3, 700, 31), (1, 1000, 33), (2, 1300, 24 * 8), (5, 1, 40),
@@ -220,6 +220,30 @@ def test_overrun_poisons_and_is_counted(op):
         assert torch.isnan(a[:, 2 * steps:10 * steps]).all()
         nan = torch.isnan(a)
         assert bits_equal(a[~nan], b[~nan])
+
+
+# rows of 1 to 3 vectors: one tile of up to 2048 steps; several of 512 steps while all are resident
+# (1024 workgroups in the forward, 768 in the backward) and a chain has at most 32; longer ones otherwise
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("shape,vectors", [((4, 2048), 1), ((4, 2049), 1), ((2, 16384), 1),
+                                           ((2, 16385), 1), ((3, 1025), 2), ((3, 681), 3),
+                                           ((204, 2049), 1), ((154, 2049), 1), ((205, 2049), 1)],
+                         ids=str)
+def test_narrow_rows(shape, vectors, dtype):
+    test_short_sequences(dtype, (*shape, vectors))
+
+
+@pytest.mark.parametrize("seqlen,steps", [(2049, 512), (16384, 512), (16385, 1024)])
+def test_narrow_rows_take_short_tiles(seqlen, steps):
+    """Tile 1 never publishes: the first value that its silence makes NaN is tile 2's."""
+    g, x = (torch.rand(1, seqlen, 4, device=DEVICE) for _ in range(2))
+    ops.set_lookback_test_hook(1, 64)
+    try:
+        y = fpscan_amd.scan_forward_channel_last(g, x)
+        torch.cuda.synchronize()
+    finally:
+        ops.set_lookback_test_hook()
+    assert torch.isnan(y[0, :, 0]).nonzero()[0].item() == 2 * steps
 
 
 # the sizes from which the ring of tiles takes over: split rows on 64-byte lines below and from 192

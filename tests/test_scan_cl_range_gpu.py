@@ -15,7 +15,7 @@ pytestmark = [
 ]
 
 # (batch, seqlen, 16-byte vectors per row): on the 128-byte lines, one tile and 11, few chains and 48
-# (the backward's two tile lengths); off the lines, rows of 1 vector (tiles of 2048 steps) and 9
+# (the backward's two tile lengths); off the lines, rows of 1 vector (tiles of 512 steps) and 9
 SHAPES = [(1, 250, 8), (2, 2600, 8), (2, 1100, 24 * 8), (2, 6000, 1), (1, 2600, 9)]
 
 
