@@ -1512,7 +1512,17 @@ constexpr int64_t kClKeepMaxBytes = 128ll << 20;
 // 145, f16 (782, 187, 184) 36 + 64 -> 46 + 71; wider rows with a last tile that is half empty lose,
 // bf16 (512, 257, 520) 105 + 182 -> 127 + 213, (128, 257, 2056) 116 + 192 -> 125 + 205, and with full
 // tiles are even, (64, 512, 4104) 201 + 356 -> 201 + 357.
+// The forward of rows of 20 to 32 vectors keeps the one pass where its waves fill the CUs evenly, three or
+// four on each: bf16 (750, 512, 208) 94 -> 112, (750, 1400, 232) 282 -> 318, (701, 512, 248) 102 -> 120,
+// (1005, 362, 248) 112 -> 121, fp32 (750, 512, 104) 96 -> 107, (946, 512, 92) 107 -> 114. With 520
+// sequences, two on most CUs and three on some, blocks are 2-40 % faster up to 26 vectors and within 3 %
+// above, bf16 (520, 1000, 184) 142 -> 132, (520, 2000, 232) 312 -> 320, fp32 (520, 512, 80) 74 -> 46;
+// with 1100 and more even on average, bf16 (1100, 1000, 184) 288 -> 271, fp32 (1600, 512, 92) 194 ->
+// 187, (1100, 1000, 80) 215 -> 223. The backward there, (757, 700, 168) to (701, 512, 248), is 4 % slower
+// to 5 % faster.
 constexpr int64_t kClbNarrow = 16;
+constexpr int64_t kClbEvenVectors = 20;
+constexpr int64_t kClbEvenMin = 576, kClbEvenMax = 1024;
 constexpr int64_t kClbNarrowSteps = 256;
 
 // Taken in the automatic mode where one pass per strip lacks strips, whatever the size when
@@ -1593,7 +1603,11 @@ ClBlockPlan plan_cl_blocks(int64_t batch, int64_t seqlen, int64_t dim, int64_t s
     return t;
   } else if (enough_strips) {
     if (t.nseg < 2) return t;
-    const bool narrow = nv <= kClbNarrow || (nv <= kClbMaxCv && seqlen >= kClbNarrowSteps);
+    // below 33 vectors a sequence is one strip
+    const bool even =
+        !bwd && nv >= kClbEvenVectors && batch >= kClbEvenMin && batch <= kClbEvenMax;
+    const bool narrow =
+        nv <= kClbNarrow || (nv <= kClbMaxCv && seqlen >= kClbNarrowSteps && !even);
     if (bytes < kClTiledMinBytes && !narrow) return t;
   }
   t.use = true;

@@ -114,3 +114,26 @@ def test_steps_of_the_channel_last_backward(dtype, seqlen, chains, steps):
     gg_ref, gx_ref = oracle.scan_bwd_f64_channel_last(*(t[..., pick].cpu() for t in (g, y, go)))
     check(gx[..., pick].cpu(), gx_ref, dtype, "grad_tokens")
     check(gg[..., pick].cpu(), gg_ref, dtype, "grad_gates")
+
+
+# off the lines with enough strips: the forward of rows of 20 to 32 vectors takes the one pass with 576
+# to 1024 sequences, blocks around that and on fewer vectors; the backward always blocks
+@pytest.mark.parametrize("batch,vectors,fwd", [(575, 21, "scan_cl_blocks"), (576, 20, "scan_cl"),
+                                               (1024, 31, "scan_cl"), (1025, 20, "scan_cl_blocks"),
+                                               (700, 19, "scan_cl_blocks")], ids=str)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+def test_kernel_of_narrow_rows_with_enough_strips(dtype, batch, vectors, fwd):
+    shape = (batch, 260, vectors * (16 // torch.empty((), dtype=dtype).element_size()))
+    g = (0.9 + 0.09 * torch.rand(shape, device=DEVICE)).to(dtype)
+    x, go = (torch.randn(shape, device=DEVICE).to(dtype) for _ in range(2))
+    for reverse in (False, True):
+        assert kernels(lambda: fpscan_amd.scan_forward_channel_last(g, x, reverse))[-1][0] == fwd
+    y = fpscan_amd.scan_forward_channel_last(g, x)
+    at = [t[-1:].cpu() for t in (g, x, go, y)]
+    check(at[3], oracle.scan_f64_channel_last(at[0], at[1]), dtype, "forward")
+    run = lambda: fpscan_amd.scan_backward_channel_last(g, y, go)  # noqa: E731
+    assert kernels(run)[-1][0] == "scan_cl_blocks"
+    gg_ref, gx_ref = oracle.scan_bwd_f64_channel_last(at[0], at[3], at[2])
+    gg, gx = run()
+    check(gx[-1:].cpu(), gx_ref, dtype, "grad_tokens")
+    check(gg[-1:].cpu(), gg_ref, dtype, "grad_gates")
