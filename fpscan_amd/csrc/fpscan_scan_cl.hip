@@ -1501,6 +1501,13 @@ constexpr int64_t kClbMaxBytesHalfBwd = 512ll << 20;
 // 271 -> 154 + 261, but (12, 2870, 2976) 196 MiB 136 + 240 -> 140 + 243 and (4, 3964, 1184) 36 MiB 33 +
 // 53 -> 39 + 57.
 constexpr int64_t kClbMaxBytesHalfLines = 192ll << 20;
+// There the fp32 backward with 48 chains or more, whose forward stays with blocks, from 96 MiB, blocks ->
+// tiles: (24, 1092, 240) 128 MiB, 192 chains, 11 % faster, (8, 3640, 1200) 304 chains 12 %, (8, 4369, 240),
+// 96 MiB 8 %, (24, 364, 1200) 8 %, (4, 7447, 880) 112 chains 8 %, but 40 MiB 30-40 % slower, and with
+// fewer chains, (2, 14895, 880) 56 at 96 MiB, (2, 32768, 400) 26 at 100 MiB, 1-6 % slower; the 2-byte
+// backward is even on average.
+constexpr int64_t kClbMaxBytesHalfLinesF32Bwd = 96ll << 20;
+constexpr int64_t kClbHalfLinesChains = 48;
 // The largest tensor whose gates and output the forward of a training step keeps (as for rows).
 constexpr int64_t kClKeepMaxBytes = 128ll << 20;
 
@@ -1599,7 +1606,10 @@ ClBlockPlan plan_cl_blocks(int64_t batch, int64_t seqlen, int64_t dim, int64_t s
   if (!t.shared) {
     const bool half_bwd = bwd && size == 2 && t.chains > 16 && t.chains < 128;
     if (enough_strips || bytes >= (half_bwd ? kClbMaxBytesHalfBwd : kClbMaxBytes)) return t;
-  } else if (t.npan > 1 && (stride_t * size) % 64 == 0 && bytes >= kClbMaxBytesHalfLines) {
+  } else if (t.npan > 1 && (stride_t * size) % 64 == 0 &&
+             bytes >= (bwd && size == 4 && t.chains >= kClbHalfLinesChains
+                           ? kClbMaxBytesHalfLinesF32Bwd
+                           : kClbMaxBytesHalfLines)) {
     return t;
   } else if (enough_strips) {
     if (t.nseg < 2) return t;

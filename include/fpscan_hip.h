@@ -166,7 +166,8 @@ size_t fpscan_workspace_bytes(int64_t batch, int64_t dim, int64_t seqlen, int dt
  *   than 512 strips of 64 16-byte vectors (batch * ceil(dim / (64 * 16/itemsize))) below 1 GiB per
  *   tensor (512 MiB in the 2-byte backward with 17 to 127 panels), except sequences of a few
  *   steps; and where rows (stride_t * itemsize) are not whole 128-byte lines at any size, but for
- *   rows on 64-byte lines of several panels from 192 MiB, and with 512 strips or more
+ *   rows on 64-byte lines of several panels from 192 MiB (the fp32 backward with 48 panels or more
+ *   from 96), and with 512 strips or more
  *   below 512 MiB only on narrow rows (16 vectors, 32 from 256 steps but for the forward of 20 and
  *   more with 576 to 1024 sequences). A sequence within one tile uses no workspace.
  * - tiles of 64 columns by 128 steps (64 in fp32) with a look-back, on a persistent grid: fewer

@@ -137,3 +137,23 @@ def test_kernel_of_narrow_rows_with_enough_strips(dtype, batch, vectors, fwd):
     gg, gx = run()
     check(gx[-1:].cpu(), gx_ref, dtype, "grad_tokens")
     check(gg[-1:].cpu(), gg_ref, dtype, "grad_gates")
+
+
+# split rows on 64-byte lines: the fp32 backward with 48 chains (panels of 8 vectors) or more takes the
+# ring of tiles from 96 MiB, the forward and fewer chains from 192 MiB
+@pytest.mark.parametrize("shape,bwd", [((8, 13107, 240), "scan_cl_blocks"),
+                                       ((8, 13108, 240), "scan_cl_tiles"),
+                                       ((6, 17477, 240), "scan_cl_tiles"),
+                                       ((5, 20972, 240), "scan_cl_blocks")], ids=str)
+def test_kernel_of_the_fp32_backward_on_64_byte_lines(shape, bwd):
+    g = 0.9 + 0.09 * torch.rand(shape, device=DEVICE)
+    x, go = (torch.randn(shape, device=DEVICE) for _ in range(2))
+    assert kernels(lambda: fpscan_amd.scan_forward_channel_last(g, x))[-1][0] == "scan_cl_blocks"
+    y = fpscan_amd.scan_forward_channel_last(g, x)
+    run = lambda: fpscan_amd.scan_backward_channel_last(g, y, go)  # noqa: E731
+    assert kernels(run)[-1][0] == bwd
+    gg, gx = run()
+    at = [t[-1:, :, [0, -1]].cpu() for t in (g, y, go, gg, gx)]
+    gg_ref, gx_ref = oracle.scan_bwd_f64_channel_last(*at[:3])
+    check(at[4], gx_ref, torch.float32, "grad_tokens")
+    check(at[3], gg_ref, torch.float32, "grad_gates")
